@@ -234,6 +234,7 @@ hipError_t prepare_gemv() {
     if (e == hipSuccess)
       e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)gemv_tern_lds_bytes(kGemvMaxK));
+  if (e == hipSuccess) e = prepare_gemv_batch();
   return e;
 }
 
@@ -245,6 +246,7 @@ hipError_t launch_hadamard(const float *x, int64_t ldx, const float *signs, floa
 }
 
 hipError_t launch_gemv(const GemvArgs &g, hipStream_t stream, hipEvent_t *ev, hipEvent_t done) {
+  if (g.tab) return launch_gemv_batch(g, stream, ev, done);
   const bool two = g.nru == 2;
   switch (g.type) {
     case kW_F32: return two ? launch_fmt<kW_F32, 2>(g, stream, ev, done) : launch_fmt<kW_F32, 1>(g, stream, ev, done);

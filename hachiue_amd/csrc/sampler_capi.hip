@@ -187,6 +187,7 @@ struct hs_context {
   DevBuf split_list, split_meta, split_cnt;   // split rows (split_cnt: zero between calls)
   DevBuf gemv_part, gemv_cnt;   // Q4_K/Q6_K GEMV tiles cut between waves (gemv_cnt: zero between calls)
   DevBuf gemv_rot;              // the Hadamard-rotated input of a folded weight
+  DevBuf gemv_tab;              // limb tables of several activation rows (one size, for good)
   DevBuf fuse_rows, fuse_pool, fuse_hist;   // lm_head GEMV that samples its rows: counters
                                 //   (zero between calls), the waves' two largest, the
                                 //   rows' key histograms (zero between calls)
@@ -756,7 +757,21 @@ int gemv_setup(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, const 
   const int64_t wpb = hs::kGemvThreads / 64;
   g.blocks = (int32_t)std::min<int64_t>((steps + wpb - 1) / wpb, 1 << 20);
   if (M > 65535) return fail(HS_ERR_UNSUPPORTED, "M %d above 65535", M);
-  if (w_type == hs::kW_Q6_K || w_type == hs::kW_Q4_K) {   // the hand-over slots of tiles cut between waves
+  if (hs::gemv_batched(w_type, M)) {
+    // several rows: their limb tables (one allocation of the largest size, so
+    // that a captured graph's address stays good).  A first call that is
+    // being captured cannot allocate and takes a row at a time.
+    if (!ctx->gemv_tab.p) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(stream, &cs) != hipSuccess) {
+        (void)hipGetLastError();
+        cs = hipStreamCaptureStatusActive;
+      }
+      if (cs == hipStreamCaptureStatusNone) HS_HIP(ctx->gemv_tab.ensure(hs::kBatchTabBytes));
+    }
+    g.tab = ctx->gemv_tab.p;
+  }
+  if (!g.tab && (w_type == hs::kW_Q6_K || w_type == hs::kW_Q4_K)) {   // the hand-over slots of tiles cut between waves
     int cus = 0;
     HS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
     g.part_cap = cus * hs::kGemvWavesPerCU;
@@ -1187,6 +1202,7 @@ int hs_context_destroy(hs_context *ctx) {
     ctx->gemv_part.release();
     ctx->gemv_cnt.release();
     ctx->gemv_rot.release();
+    ctx->gemv_tab.release();
     ctx->large_retry.release();
     ctx->large_replay.release();
     ctx->replay_slots.release();
@@ -1294,7 +1310,9 @@ int lm_head_sample(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, co
   // (HS_LMHEAD_FUSE=2): their argmax launch measured 2.7 us (no penalty) to
   // 9 us (repetition penalty) slower than the GEMV and the argmax launch
   const bool sample_ok = tern || w->type == hs::kW_Q6_K || w->type == hs::kW_Q4_K;
+  // (several rows whose GEMV reads the weights once for all of them: two launches)
   bool fused = ctx->fuse && (sample_ok || ctx->fuse >= 2) && M > 0 && w->rows > 0 && configs &&
+               !hs::gemv_batched(w->type, M) &&
                d_uniforms && d_tokens && (d_hist_ids == nullptr) == (d_hist_offsets == nullptr);
   std::vector<hs::RowPlan> plans;
   Routing rt;

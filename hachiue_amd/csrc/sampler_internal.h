@@ -232,6 +232,9 @@ struct GemvArgs {
   // block scales (N * K / 128 of each), s_bytes their size
   const void *scales;
   uint32_t s_bytes;
+  // several activation rows in one pass over the weights (batch_gemv.hip):
+  // the workspace of their limb tables, or null for a row at a time
+  void *tab;
 };
 // The 512-wide Hadamard rotation of a hadamard-folded weight's input
 // (src/kernels.ts:177-227, mode 0): out[m][k] for m < M, k < K (K a multiple
@@ -252,6 +255,16 @@ constexpr int gemv_batch_chunks(int type) {
 constexpr int gemv_lds_bytes(int type) { return (kGemvThreads / 64) * gemv_batch_chunks(type) * 1024; }
 hipError_t launch_gemv(const GemvArgs &g, hipStream_t stream, hipEvent_t *ev, hipEvent_t done);
 hipError_t prepare_gemv();      // per device, once (called by prepare_kernels)
+// Several activation rows in one pass over the weights (batch_gemv.hip), the
+// rows of one launch, and the bytes of their limb tables (16 slices of 16
+// rows, K / 256 blocks of at most 17152 bytes each).
+constexpr int kBatchRows = 256;
+constexpr size_t kBatchTabBytes = (size_t)(kBatchRows / 16) * (kGemvMaxK / 256) * 17152;
+constexpr bool gemv_batched(int type, int M) {
+  return M >= 2 && (type == kW_Q6_K || type == kW_Q4_K);
+}
+hipError_t launch_gemv_batch(GemvArgs g, hipStream_t stream, hipEvent_t *ev, hipEvent_t done);
+hipError_t prepare_gemv_batch();   // per device, once (called by prepare_gemv)
 
 // ---- decode step bookkeeping (after the sampler, same stream)
 struct DecodeArgs {
