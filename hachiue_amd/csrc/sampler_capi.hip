@@ -160,7 +160,7 @@ constexpr size_t pin_align(size_t b) { return (b + 255) / 256 * 256; }
 
 // Routing of rows to kernels, uploaded next to the plans.
 struct Routing {
-  std::vector<int32_t> pf, row, chunk, large, mid, lfast;
+  std::vector<int32_t> pf, row, chunk, large, mid, lfast, minp;
 };
 
 std::mutex g_prep_mu;
@@ -196,6 +196,7 @@ struct hs_context {
   // for calls with k <= 64 sampling rows there and all-greedy calls on the
   // vector-unit weights (F32, Q4_0, Q4_1)
   int fuse = 1;
+  DevBuf minp_cand, minp_meta;  // split min-p rows' hand-over (counted in by split_cnt)
   DevBuf large_retry;           // two-pass large-k rows handed back
   DevBuf large_replay;          // slot-history replays asked for by the large-k kernel
   DevBuf replay_slots;          // the device-memory replay's regions: keys, then ids
@@ -287,6 +288,11 @@ bool two_pass_large(const hs::RowPlan &p, int vocab) {
   return p.mode == hs::kModeLarge && p.k >= vocab && !(p.min_p > 0.0);
 }
 
+// k = vocab with a min-p that leaves few candidates: the min-p kernel's rows.
+bool minp_large(const hs::RowPlan &p, int vocab) {
+  return p.mode == hs::kModeLarge && p.k >= vocab && p.min_p >= hs::kMinpLeast && vocab < (1 << 26);
+}
+
 // One row's plan: the `??`-resolved config of src/sampler.ts:18-22 with k
 // resolved (:49) and the kernel mode.
 hs::RowPlan plan_row(const hs_sample_config &c, int vocab) {
@@ -330,11 +336,12 @@ int build_plans(const hs_sample_config *cfgs, int rows, int vocab, int row_min_r
   rt.large.clear();
   rt.mid.clear();
   rt.lfast.clear();
+  rt.minp.clear();
   for (int r = 0; r < rows; ++r) {
     const hs::RowPlan p = plan_row(cfgs[r], vocab);
     out[(size_t)r] = p;
     if (p.mode == hs::kModeLarge) {
-      (two_pass_large(p, vocab) ? rt.lfast : rt.large).push_back(r);
+      (two_pass_large(p, vocab) ? rt.lfast : minp_large(p, vocab) ? rt.minp : rt.large).push_back(r);
       continue;
     }
     const bool one_pass = vocab <= hs::kRowMaxVocab && rows >= row_min_rows;
@@ -364,7 +371,7 @@ int upload_plans(hs_context *ctx, const std::vector<hs::RowPlan> &plans, const R
   const size_t pbytes = rows * sizeof(hs::RowPlan);
   const size_t lbytes =
       sizeof(int32_t) * (rt.pf.size() + rt.row.size() + rt.chunk.size() + rt.large.size() +
-                         rt.mid.size() + rt.lfast.size());
+                         rt.mid.size() + rt.lfast.size() + rt.minp.size());
   const size_t bytes = pbytes + lbytes;
   if (ctx->last_plans.size() == rows && ctx->last_vocab == vocab && ctx->plans.bytes >= bytes &&
       memcmp(ctx->last_plans.data(), plans.data(), pbytes) == 0)
@@ -385,7 +392,8 @@ int upload_plans(hs_context *ctx, const std::vector<hs::RowPlan> &plans, const R
   memcpy(st, plans.data(), pbytes);
   int32_t *lists = reinterpret_cast<int32_t *>(st + pbytes);
   // the lists back to back (an empty list's data() may be null: no copy)
-  for (const std::vector<int32_t> *l : {&rt.pf, &rt.row, &rt.chunk, &rt.large, &rt.mid, &rt.lfast}) {
+  for (const std::vector<int32_t> *l : {&rt.pf, &rt.row, &rt.chunk, &rt.large, &rt.mid, &rt.lfast,
+                                        &rt.minp}) {
     if (!l->empty()) memcpy(lists, l->data(), sizeof(int32_t) * l->size());
     lists += l->size();
   }
@@ -535,7 +543,7 @@ int sample_device(hs_context *ctx, float *d_logits, int32_t rows, int64_t row_st
   }
   const int n_pf = (int)rt.pf.size(), n_row = (int)rt.row.size(), n_chunk = (int)rt.chunk.size();
   const int n_large = (int)rt.large.size(), n_mid = (int)rt.mid.size();
-  const int n_lfast = (int)rt.lfast.size();
+  const int n_lfast = (int)rt.lfast.size(), n_minp = (int)rt.minp.size();
 
   // workspace (the chunk path only)
   if (n_chunk > 0) {
@@ -563,6 +571,18 @@ int sample_device(hs_context *ctx, float *d_logits, int32_t rows, int64_t row_st
   const int split = choose_split(ctx, n_row, vocab);
   int rc = ensure_split(ctx, n_row, split, stream);
   if (rc) return rc;
+  // so does the min-p kernel (whole rows where the general path takes them:
+  // unaligned ones and calls that want candidates)
+  const bool vec = (reinterpret_cast<uintptr_t>(d_logits) & 15u) == 0 && (row_stride & 3) == 0;
+  const bool want_cands = d_cand_ids || d_cand_probs;
+  const int minp_split = vec && !want_cands ? choose_split(ctx, n_minp, vocab) : 1;
+  if (minp_split > 1) {
+    const size_t parts = (size_t)n_minp * (size_t)minp_split;
+    HS_HIP(ctx->minp_cand.ensure(parts * hs::kMinpHand * sizeof(unsigned long long)));
+    HS_HIP(ctx->minp_meta.ensure(parts * sizeof(hs::MinpMeta)));
+    rc = ensure_zeroed(ctx->split_cnt, sizeof(uint32_t) * (size_t)n_minp, stream);
+    if (rc) return rc;
+  }
   rc = upload_plans(ctx, plans, rt, vocab, stream);
   if (rc) return rc;
 
@@ -575,6 +595,9 @@ int sample_device(hs_context *ctx, float *d_logits, int32_t rows, int64_t row_st
   ws.large_list = lists + n_pf + n_row + n_chunk;
   ws.mid_list = lists + n_pf + n_row + n_chunk + n_large;
   ws.lfast_list = lists + n_pf + n_row + n_chunk + n_large + n_mid;
+  ws.minp_list = ws.lfast_list + n_lfast;
+  ws.minp_cand = static_cast<unsigned long long *>(ctx->minp_cand.p);
+  ws.minp_meta = static_cast<hs::MinpMeta *>(ctx->minp_meta.p);
   ws.large_retry = static_cast<int32_t *>(ctx->large_retry.p);
   ws.large_replay = static_cast<hs::ReplayReq *>(ctx->large_replay.p);
   if (replay_dev > 0) {
@@ -593,8 +616,8 @@ int sample_device(hs_context *ctx, float *d_logits, int32_t rows, int64_t row_st
   a.rows = rows;
   a.vocab = vocab;
   a.chunks = (int32_t)S;
-  a.vec = ((reinterpret_cast<uintptr_t>(d_logits) & 15u) == 0 && (row_stride & 3) == 0) ? 1 : 0;
-  a.want_cands = (d_cand_ids || d_cand_probs) ? 1 : 0;
+  a.vec = vec ? 1 : 0;
+  a.want_cands = want_cands ? 1 : 0;
   a.n_pf = n_pf;
   a.n_row = n_row;
   a.split = split;
@@ -603,6 +626,8 @@ int sample_device(hs_context *ctx, float *d_logits, int32_t rows, int64_t row_st
   a.n_large = n_large;
   a.n_mid = n_mid;
   a.n_lfast = n_lfast;
+  a.n_minp = n_minp;
+  a.minp_split = minp_split;
   a.replay_dev = replay_dev;
   a.hist_ids = d_hist_ids;
   a.hist_off = d_hist_offsets;
@@ -1203,6 +1228,8 @@ int hs_context_destroy(hs_context *ctx) {
     ctx->gemv_cnt.release();
     ctx->gemv_rot.release();
     ctx->gemv_tab.release();
+    ctx->minp_cand.release();
+    ctx->minp_meta.release();
     ctx->large_retry.release();
     ctx->large_replay.release();
     ctx->replay_slots.release();

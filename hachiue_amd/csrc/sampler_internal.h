@@ -58,7 +58,7 @@ enum RowMode : int32_t {
   kModeGreedy = 0,   // temperature <= 0 (src/sampler.ts:36-46)
   kModeSmall = 1,    // 1 <= k <= 64
   kModeGeneric = 2,  // 64 < k <= 1024
-  kModeLarge = 3,    // k > 1024 (large_kernel)
+  kModeLarge = 3,    // k > 1024 (minp_kernel, large_fast_kernel, large_kernel)
 };
 
 enum RowPen : int32_t {
@@ -124,6 +124,21 @@ constexpr int kReplayDevMaxK = 1 << 24;
 constexpr int kReplayDevCands = 8192;
 constexpr int kReplayDevBlocks = 16;
 
+// min-p rows with k = vocab (minp_kernel): the least min_p it is given (below,
+// the candidates are often more than it sorts and the general path, which
+// then finishes the row, is taken at once), the candidates a part hands over,
+// and what else it does.
+constexpr double kMinpLeast = 1.0 / 256;
+constexpr int kMinpHand = 1024;
+struct MinpMeta {
+  unsigned long long s;      // (binary64 bits) sum of exp((v - m) / T), m the part's maximum
+  uint32_t mkey;             // key of m, 0: no logit above -Infinity
+  uint32_t nf;               // logits above -Infinity
+  int32_t count;             // candidates handed over, -1: too many
+  uint32_t pad;
+};
+static_assert(sizeof(MinpMeta) == 24, "MinpMeta layout");
+
 struct Workspace {
   RowPlan *plans;            // [rows]
   const int32_t *pf_list;    // rows penalised by the pre-pass
@@ -132,6 +147,9 @@ struct Workspace {
   const int32_t *large_list; // rows of the large-k kernel
   const int32_t *mid_list;   // rows of the mid kernel
   const int32_t *lfast_list; // rows of the two-pass large-k kernel (k = vocab, no min-p)
+  const int32_t *minp_list;  // rows of the min-p kernel
+  unsigned long long *minp_cand;    // [n_minp][minp_split][kMinpHand] packed candidates
+  MinpMeta *minp_meta;              // [n_minp][minp_split]
   int32_t *large_retry;      // [n_lfast] 1: the two-pass kernel handed the row back
   ReplayReq *large_replay;   // [n_large] slot-history replays asked for by large_row
   uint32_t *replay_keys;     // [replay_dev][vocab] slots of the device-memory replay
@@ -142,7 +160,7 @@ struct Workspace {
   ChunkInfo *info;           // [n_chunk][S]
   unsigned long long *split_list;   // [n_row][split][kPartCap] packed candidates
   SplitMeta *split_meta;            // [n_row][split]
-  uint32_t *split_cnt;              // [n_row] parts arrived (0 between calls)
+  uint32_t *split_cnt;              // [n_row or n_minp] parts arrived (0 between calls)
 };
 
 struct LaunchArgs {
@@ -156,6 +174,8 @@ struct LaunchArgs {
   int32_t rows_direct;       // the row kernel takes every row: row = block index
   int32_t n_pf, n_row, n_chunk, n_large, n_mid;
   int32_t n_lfast;           // rows of the two-pass large-k kernel
+  int32_t n_minp;            // rows of the min-p kernel, and its workgroups per row
+  int32_t minp_split;
   int32_t n_argmax;          // rows of the GPU greedy route (a call of its own)
   int32_t split;             // row / argmax kernel: workgroups per row (1: whole rows)
   int32_t replay_dev;        // workgroups of the device-memory slot replay (0: not launched)
@@ -184,16 +204,16 @@ struct LaunchArgs {
 // ev[2i] and ev[2i + 1] receive the start and end of kernel i's dispatch
 // (0 penalty pre-pass, 1 row kernel, 2 chunk kernel, 3 finalize, 4 large-k
 // kernel, 5 mid kernel, 6 GPU greedy-route argmax, 8 two-pass large-k kernel,
-// 9 the large-k slot replay, 10 the device-memory slot replay;
+// 9 the large-k slot replay, 10 the device-memory slot replay, 11 min-p kernel;
 // 7 is the lm_head GEMV, launched apart), for the kernels that launch only:
 // launched_kernels() says which.  The large-k kernel launches whenever a row
 // has k > 1024: it also takes the rows the two-pass kernel hands back.
-constexpr int kTimedKernels = 11;
+constexpr int kTimedKernels = 12;
 inline unsigned launched_kernels(const LaunchArgs &a) {
   return (a.n_pf > 0 ? 1u : 0u) | (a.n_row > 0 ? 2u : 0u) | (a.n_chunk > 0 ? 12u : 0u) |
          (a.n_large + a.n_lfast > 0 ? 16u : 0u) | (a.n_mid > 0 ? 32u : 0u) |
          (a.n_argmax > 0 ? 64u : 0u) | (a.n_lfast > 0 ? 256u : 0u) | (a.n_large > 0 ? 512u : 0u) |
-         (a.n_large > 0 && a.replay_dev > 0 ? 1024u : 0u);
+         (a.n_large > 0 && a.replay_dev > 0 ? 1024u : 0u) | (a.n_minp > 0 ? 2048u : 0u);
 }
 // Largest vocabulary of the GPU greedy route (byte offsets of a row stay
 // below 2^31).

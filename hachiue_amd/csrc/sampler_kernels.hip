@@ -31,7 +31,9 @@
 //                    list.
 //   finalize_kernel  one workgroup per chunk-kernel row: exact select over the
 //                    row's candidates, then the shared row completion.
-//   large_kernel     rows with k > 1024: one 1024-thread workgroup per row,
+//   minp_kernel      rows with k = vocab and min-p: one pass, split like the
+//                    row kernel's rows.
+//   large_kernel     the other rows with k > 1024: one 1024-thread workgroup per row,
 //                    several passes (radix select of the k-th value, softmax
 //                    normaliser, probability-mass histogram, positions located
 //                    by narrowing one bucket).
@@ -5600,6 +5602,341 @@ __global__ __launch_bounds__(kLT) void large_kernel(LaunchArgs a, Workspace ws) 
   large_row(a, P, row, *reinterpret_cast<LargeSmem *>(ldyn), req);
 }
 
+// ---------------------------------------------------------------- min-p, one pass
+
+// Rows with k = vocab and min-p (min_p >= kMinpLeast): no slot is evicted, so
+// the order is value descending, index ascending, and only the candidates of
+// probability at least min_p times the largest can be drawn, those at or above
+// max + T ln(min_p): usually a few.  One pass over the row collects them and
+// sums the normaliser; the rest runs on the collected list.
+//
+//  - A row is split over a.minp_split workgroups like the row kernel's; the
+//    parts stream it in rounds of kMpNV float4 per thread, two in flight.
+//  - Every wave keeps its own maximum m_w, raised before a round is summed
+//    (its sums are then scaled down), so no weight 2^((v - m_w) log2(e) / T)
+//    exceeds 1; they are added up in binary64.  The exponent is the binary32
+//    product with log2(e) / T as two binary32 parts, so that only roundings
+//    of its own, not one shared by the whole row, remain.
+//  - Logits at or above max so far + T ln(min_p) (a little less: kMpSlack)
+//    go to a list in LDS; the maximum is shared by the waves through LDS.
+//  - A part hands over its sums, its maximum and the listed logits that its
+//    final bound keeps; the last part merges them, sorts the list (it holds
+//    every candidate of min-p, and the row's maximum) and takes the
+//    reference's probabilities f32(f32(exp((v - m) / T)) / S), the min-p and
+//    top-p stops and the draw from it (src/sampler.ts:83-117).
+// A row this does not suit (more than kMpCap logits listed by a part or
+// kSortCap kept, an infinite maximum, a normaliser that is not finite,
+// unaligned rows, candidate outputs) is finished by large_row instead, by the
+// same workgroup.
+// Bound: one read of the row; the general path reads it four to six times
+// with one workgroup per row.  50 rows x 151936, min-p 0.05, repetition 1.1:
+// 174 us a call before (the general path 161 us of it), 30 us now (pen_kernel
+// 6, this kernel 25).
+constexpr int kMpNV = 8;          // float4 per thread and round
+constexpr int kMpCap = 4096;      // logits a part lists
+constexpr double kMpSlack = 1e-5; // of T, below the bound (probabilities round at 2^-24)
+
+struct MinpSmem {
+  unsigned long long list[kMpCap];   // then the sorted list's cumulative sums
+  unsigned long long srt[kSortCap];
+  unsigned long long tmp[kSortCap];
+  uint32_t cnt[kBinSortBins + 32];
+  double dred[kRowWaves];
+  uint32_t wkey[kRowWaves], wnf[kRowWaves];
+  double s;                          // the part's, then the row's normaliser
+  uint32_t mkey, nf;                 // its maximum (key), logits above -Infinity
+  uint32_t mx;                       // largest key seen so far by any wave
+  int32_t nlist, nsrt, last, bad, f1, f2, pick;
+  int32_t pcnt[kSplitMax];           // the parts' list lengths
+};
+size_t minp_smem_bytes() {
+  return sizeof(MinpSmem) > sizeof(LargeSmem) ? sizeof(MinpSmem) : sizeof(LargeSmem);
+}
+
+// One part of a row (and the row itself, in its last part); false: the row
+// goes to large_row.
+__device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &ws, const RowPlan &P,
+                                         int row, int slot, int part, MinpSmem &sm) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = uniform_i32(tid >> 6);
+  const int S = a.minp_split;
+  const float *rowp = a.logits + (int64_t)row * a.stride;
+  const int nfull = a.vocab >> 2, per = (nfull + S - 1) / S;
+  const int f0 = min(nfull, part * per), n4 = min(nfull, f0 + per) - f0;
+  const rsrc_t r4 = make_rsrc(rowp + 4 * (int64_t)f0, 16u * (uint32_t)n4);
+  f32x4 A[kMpNV], B[kMpNV];
+  auto load = [&](f32x4 (&t)[kMpNV], int fb) {
+#pragma unroll
+    for (int u = 0; u < kMpNV; ++u) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b128(r4, (fb + u * kRowThreads + tid) * 16, 0, kReadNT);
+      t[u] = f32x4{__uint_as_float(x[0]), __uint_as_float(x[1]), __uint_as_float(x[2]),
+                   __uint_as_float(x[3])};
+    }
+  };
+  constexpr int kRound = kMpNV * kRowThreads;
+  load(A, 0);
+  load(B, kRound);
+  __builtin_amdgcn_sched_barrier(0);
+  // the logits past the row's last whole float4, one each for the last
+  // part's first threads
+  const int et = 4 * nfull + tid;
+  const bool has_tail = part == S - 1 && tid < (a.vocab & 3);
+  const float vt = has_tail ? rowp[et] : -INFINITY;
+  const double u01 = load_scalar(a.uniforms + row);
+  if (tid == 0) {
+    sm.mx = 0;
+    sm.nlist = sm.nsrt = sm.f1 = sm.bad = 0;
+    sm.f2 = sm.pick = 0x7FFFFFFF;
+  }
+  __syncthreads();
+  const double it = 1.0 / P.temperature;
+  const double cd = it * 1.4426950408889634074;   // log2(e) / T
+  const float ch = (float)cd, cl = (float)(cd - (double)ch);
+  const float off = (float)((P.min_p < 1.0 ? log(P.min_p) * P.temperature : 0.0) - kMpSlack * P.temperature);
+  // the list's bound for a maximum mx (the binary32 sum's rounding taken off)
+  auto bound = [&](float mx) { return (mx + off) - 2.4e-7f * (fabsf(mx) + fabsf(off)); };
+
+  float m_w = -INFINITY;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  uint32_t nf = 0;
+  auto append = [&](float v, int e, bool ok) {
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
+    if (m == 0ull) return;
+    int base = 0;
+    if (lane == 0) base = atomicAdd(&sm.nlist, __popcll(m));
+    base = __builtin_amdgcn_readfirstlane(base);
+    const int p = base + (int)lanes_below(m);
+    if (ok && p < kMpCap) sm.list[p] = pack_cand(f2key(v), (uint32_t)e);
+  };
+  auto weigh = [&](float v, double &s) {
+    const float d = v - m_w;
+    // (NaN and -Infinity weigh 0: fmaxf gives the other operand for a NaN)
+    const float e = fmaxf(fmaf(d, ch, d * cl), -300.0f);
+    s += (double)__builtin_amdgcn_exp2f(e);
+    nf += v > -INFINITY ? 1u : 0u;
+  };
+  auto process = [&](f32x4 (&t)[kMpNV], int fb, float extra) {
+    if (fb + kRound > n4) {   // the part's last round: reads past its end do not count
+#pragma unroll
+      for (int u = 0; u < kMpNV; ++u)
+        if (fb + u * kRowThreads + tid >= n4) t[u] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    }
+    float lm = extra;
+#pragma unroll
+    for (int u = 0; u < kMpNV; ++u)
+      lm = fmaxf(lm, fmaxf(fmaxf(t[u][0], t[u][1]), fmaxf(t[u][2], t[u][3])));
+    const uint32_t wk = wave_max_u32(f2key(lm));
+    if (wk == 0u) return;   // nothing above -Infinity
+    const float wm = key2f(wk);
+    if (wm > m_w) {
+      const double f = m_w > -INFINITY ? exp(((double)m_w - (double)wm) * it) : 0.0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] *= f;
+      m_w = wm;
+      if (lane == 0) atomicMax(&sm.mx, wk);
+    }
+    const float lo = bound(key2f(__builtin_amdgcn_readfirstlane(*(volatile uint32_t *)&sm.mx)));
+    if (__builtin_expect(__any(extra > -INFINITY), 0)) {
+      weigh(extra, acc[0]);
+      append(extra, et, extra >= lo);
+    }
+#pragma unroll
+    for (int u = 0; u < kMpNV; ++u) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) weigh(t[u][c], acc[c]);
+      const bool any = t[u][0] >= lo || t[u][1] >= lo || t[u][2] >= lo || t[u][3] >= lo;
+      if (__builtin_expect(__any(any), 0)) {
+        const int e = 4 * (f0 + fb + u * kRowThreads + tid);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) append(t[u][c], e + c, t[u][c] >= lo);
+      }
+    }
+  };
+  for (int fb = 0; fb == 0 || fb < n4; fb += 2 * kRound) {
+    process(A, fb, fb == 0 ? vt : -INFINITY);
+    load(A, fb + 2 * kRound);
+    if (fb + kRound < n4) process(B, fb + kRound, -INFINITY);
+    load(B, fb + 3 * kRound);
+  }
+
+  // the part's sums: each wave's, scaled to the part's maximum
+  {
+    double sw = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    sw = wave_sum_f64(sw);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) nf += __shfl_xor(nf, d);
+    if (lane == 0) {
+      sm.dred[wave] = sw;
+      sm.wkey[wave] = f2key(m_w);
+      sm.wnf[wave] = nf;
+    }
+  }
+  __syncthreads();
+  // (lanes 0 .. n - 1 of wave 0 hold partial sums s relative to key2f(k))
+  auto combine = [&](double s, uint32_t k, uint32_t c) {
+    const uint32_t mk = wave_max_u32(k);
+    double x = k ? s * exp(((double)key2f(k) - (double)key2f(mk)) * it) : 0.0;
+    if (k == mk) x = s;   // (also where the difference is infinite minus itself)
+    x = wave_sum_f64(k ? x : 0.0);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d);
+    if (lane == 0) {
+      sm.s = x;
+      sm.mkey = mk;
+      sm.nf = c;
+    }
+  };
+  if (wave == 0)
+    combine(lane < kRowWaves ? sm.dred[lane] : 0.0, lane < kRowWaves ? sm.wkey[lane] : 0u,
+            lane < kRowWaves ? sm.wnf[lane] : 0u);
+  __syncthreads();
+  const int nl = sm.nlist;
+  bool bad = nl > kMpCap;
+  {
+    const float lo = sm.mkey ? bound(key2f(sm.mkey)) : 0.0f;
+    unsigned long long *out = S > 1 ? ws.minp_cand + (int64_t)blockIdx.x * kMinpHand : nullptr;
+    const int cap = S > 1 ? kMinpHand : kSortCap;
+    for (int i0 = 0; i0 < (bad ? 0 : nl); i0 += kRowThreads) {
+      const int i = i0 + tid;
+      const unsigned long long c = i < nl ? sm.list[i] : 0ull;
+      const bool ok = i < nl && key2f(cand_key(c)) >= lo;
+      const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
+      int base = 0;
+      if (lane == 0 && m) base = atomicAdd(&sm.nsrt, __popcll(m));
+      base = __builtin_amdgcn_readfirstlane(base);
+      const int p = base + (int)lanes_below(m);
+      if (ok && p < cap) {
+        if (S > 1) store_agent(out + p, c);
+        else sm.srt[p] = c;
+      }
+    }
+  }
+  __syncthreads();
+  if (S > 1) {
+    if (tid == 0) {
+      MinpMeta *m = ws.minp_meta + blockIdx.x;
+      store_agent(&m->s, (unsigned long long)__double_as_longlong(sm.s));
+      store_agent(&m->mkey, sm.mkey);
+      store_agent(&m->nf, sm.nf);
+      store_agent(&m->count, bad || sm.nsrt > kMinpHand ? -1 : sm.nsrt);
+    }
+    if (!split_arrive(ws, slot, S, &sm.last)) return true;
+    // the last part: every part's sums, then the lists that the row's bound
+    // keeps
+    const MinpMeta *m0 = ws.minp_meta + (int64_t)slot * S;
+    if (wave == 0) {
+      const bool in = lane < S;
+      const double s = in ? __longlong_as_double((long long)load_agent(&m0[lane].s)) : 0.0;
+      const uint32_t k = in ? load_agent(&m0[lane].mkey) : 0u;
+      const uint32_t c = in ? load_agent(&m0[lane].nf) : 0u;
+      const int n = in ? load_agent(&m0[lane].count) : 0;
+      if (in) sm.pcnt[lane] = n;
+      const bool miss = __any(n < 0);
+      combine(s, k, c);
+      if (lane == 0) {
+        sm.bad = miss ? 1 : 0;
+        sm.nsrt = 0;
+      }
+    }
+    __syncthreads();
+    bad = sm.bad != 0;
+    if (!bad) {
+      const unsigned long long *l0 = ws.minp_cand + (int64_t)slot * S * kMinpHand;
+      const float lo = sm.mkey ? bound(key2f(sm.mkey)) : 0.0f;
+      unsigned long long x[kSplitMax];
+#pragma unroll
+      for (int p = 0; p < kSplitMax; ++p)
+        x[p] = p < S && tid < sm.pcnt[p] ? load_agent(l0 + p * kMinpHand + tid) : 0ull;
+#pragma unroll
+      for (int p = 0; p < kSplitMax; ++p) {
+        const bool ok = x[p] != 0ull && key2f(cand_key(x[p])) >= lo;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
+        if (m == 0ull) continue;
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&sm.nsrt, __popcll(m));
+        base = __builtin_amdgcn_readfirstlane(base);
+        const int q = base + (int)lanes_below(m);
+        if (ok && q < kSortCap) sm.srt[q] = x[p];
+      }
+    }
+    __syncthreads();
+  }
+  const int n = sm.nsrt, n_f = (int)sm.nf;
+  const double St = sm.s;
+  const float mf = key2f(sm.mkey);
+  if (n_f <= 1 && !bad && n == n_f) {   // src/sampler.ts:76-77: no draw
+    if (tid == 0) {
+      put_token(a, row, n_f == 1 ? (int)cand_idx(sm.srt[0]) : 0);
+      if (a.cand_count_out) a.cand_count_out[row] = n_f;
+      if (a.cutoff_out) a.cutoff_out[row] = n_f;
+      if (a.row_flags) a.row_flags[row] = HS_ROW_SINGLE | HS_ROW_LARGE;
+    }
+    return true;
+  }
+  if (bad || n < 1 || n > kSortCap || !(St > 0.0 && St < INFINITY) || !(mf < INFINITY)) return false;
+  sort_binned<kRowThreads>(sm.srt, n, f2key(bound(mf)), sm.mkey, sm.cnt, sm.tmp);
+  __syncthreads();
+  double *cum = reinterpret_cast<double *>(sm.list);
+  const double thr = P.min_p * (double)(float)(1.0 / St);   // times the largest probability
+  double carry = 0.0;
+  for (int base = 0; base < n; base += kRowThreads) {
+    const int i = base + tid;
+    double p = 0.0;
+    if (i < n)
+      p = (double)(float)((double)(float)exp(((double)key2f(cand_key(sm.srt[i])) - (double)mf) * it) / St);
+    double c = wave_scan_incl_f64(p);
+    if (lane == 63) sm.dred[wave] = c;
+    __syncthreads();
+    double add = carry, tot = carry;
+    for (int w = 0; w < kRowWaves; ++w) {
+      if (w < wave) add += sm.dred[w];
+      tot += sm.dred[w];
+    }
+    c += add;
+    carry = tot;
+    if (i < n) cum[i] = c;
+    const unsigned long long keep = __builtin_amdgcn_ballot_w64(i < n && !(p < thr));
+    const unsigned long long top = __builtin_amdgcn_ballot_w64(i < n && c >= P.top_p);
+    if (lane == 0) {
+      if (keep) atomicAdd(&sm.f1, __popcll(keep));
+      if (top) atomicMin(&sm.f2, i + __builtin_ctzll(top));
+    }
+    __syncthreads();
+  }
+  // src/sampler.ts:93-105: the min-p stop, the top-p stop
+  const int f1 = sm.f1 < 1 ? 1 : sm.f1, f2 = sm.f2;
+  const int cut = f1 <= f2 ? f1 : f2 + 1;
+  // :107-116: the draw
+  const double target = u01 * cum[cut - 1];
+  for (int base = 0; base < cut; base += kRowThreads) {
+    const int i = base + tid;
+    const unsigned long long hit = __builtin_amdgcn_ballot_w64(i < cut && cum[i] >= target);
+    if (lane == 0 && hit) atomicMin(&sm.pick, i + __builtin_ctzll(hit));
+  }
+  __syncthreads();
+  if (tid == 0) {
+    // (r = u * keptSum <= 0: the first subtraction already ends the walk)
+    const int i = !(target > 0.0) && target == target ? 0 : min(sm.pick, cut - 1);
+    put_token(a, row, (int)cand_idx(sm.srt[i]));
+    if (a.cand_count_out) a.cand_count_out[row] = n_f;
+    if (a.cutoff_out) a.cutoff_out[row] = cut;
+    if (a.row_flags) a.row_flags[row] = HS_ROW_LARGE;
+  }
+  return true;
+}
+
+__global__ __launch_bounds__(kRowThreads) void minp_kernel(LaunchArgs a, Workspace ws) {
+  extern __shared__ unsigned long long ldyn[];
+  __shared__ ReplayReq unused_req;   // k = vocab: never a replay
+  const int slot = (int)blockIdx.x / a.minp_split, part = (int)blockIdx.x - slot * a.minp_split;
+  const int row = ws.minp_list[slot];
+  const RowPlan P = ws.plans[row];
+  if (a.vec && !a.want_cands) {   // (otherwise minp_split is 1)
+    if (minp_row(a, ws, P, row, slot, part, *reinterpret_cast<MinpSmem *>(ldyn))) return;
+    __syncthreads();   // (uniform: the LDS is large_row's from here)
+  }
+  large_row(a, P, row, *reinterpret_cast<LargeSmem *>(ldyn), &unused_req);
+}
+
 // ---------------------------------------------------------------- GPU greedy route
 
 // The engine sends greedy decoding without a repetition penalty
@@ -6567,6 +6904,10 @@ hipError_t prepare_kernels() {
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)replay_dev_smem_bytes())) != hipSuccess)
     return e;
+  if ((e = hipFuncSetAttribute(reinterpret_cast<const void *>(&minp_kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)minp_smem_bytes())) != hipSuccess)
+    return e;
   return hipFuncSetAttribute(reinterpret_cast<const void *>(&large_kernel),
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)large_smem_bytes());
 }
@@ -6666,7 +7007,7 @@ hipError_t launch_sample(const LaunchArgs &a, const Workspace &ws, hipStream_t s
   hipError_t e;
   // the last kernel of the call records `done`
   const int last = a.n_argmax > 0 ? 6 : a.n_large > 0 && a.replay_dev > 0 ? 10
-                 : a.n_large > 0 ? 9 : a.n_lfast > 0 ? 4
+                 : a.n_large > 0 ? 9 : a.n_lfast > 0 ? 4 : a.n_minp > 0 ? 11
                  : a.n_chunk > 0 ? 3 : a.n_mid > 0 ? 5 : a.n_row > 0 ? 1 : 0;
   auto dn = [&](int slot) { return slot == last ? done : nullptr; };
   if (a.n_pf > 0) {
@@ -6702,6 +7043,11 @@ hipError_t launch_sample(const LaunchArgs &a, const Workspace &ws, hipStream_t s
     if (e != hipSuccess) return e;
     e = launch_one(finalize_kernel, dim3((unsigned)a.n_chunk), dim3(kThreads),
                    finalize_smem_bytes(), stream, ev, 3, dn(3), a, ws);
+    if (e != hipSuccess) return e;
+  }
+  if (a.n_minp > 0) {
+    e = launch_one(minp_kernel, dim3((unsigned)(a.n_minp * a.minp_split)), dim3(kRowThreads),
+                   minp_smem_bytes(), stream, ev, 11, dn(11), a, ws);
     if (e != hipSuccess) return e;
   }
   if (a.n_lfast > 0) {

@@ -311,8 +311,8 @@ int hs_decode_step_device(hs_context *ctx, float *d_logits, int32_t rows,
  * (ms[0] presence/frequency pre-pass, ms[1] row kernel, ms[2] chunk kernel,
  * ms[3] finalize, ms[4] large-k kernel, ms[5] mid-k kernel, ms[6] greedy-route
  * argmax, ms[7] lm_head GEMV, ms[8] two-pass large-k kernel, ms[9] large-k
- * slot replay in LDS, ms[10] large-k slot replay in device memory; a kernel
- * a call did not launch adds 0)
+ * slot replay in LDS, ms[10] large-k slot replay in device memory, ms[11]
+ * min-p kernel; a kernel a call did not launch adds 0)
  * and the number of
  * timed calls, and resets the totals. */
 int hs_context_set_timing(hs_context *ctx, int enable);

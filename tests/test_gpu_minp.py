@@ -1,0 +1,95 @@
+"""GPU parity of the one-pass min-p kernel (topK >= vocab with min-p): rows
+it finishes itself, in whole rows and split over four workgroups, rows it
+gives to the general path, and the edges between them.  Tokens, cutoffs and
+counts against the oracle; a draw or top-p sum within 1e-6 of a boundary may
+differ (tests/gpu_util.py)."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_large import _check
+
+pytestmark = pytest.mark.gpu
+INF = float("inf")
+
+
+@pytest.fixture(params=["auto", "whole", "split4"])
+def ctx(request, sampler, sampler_whole, sampler_split):
+    return {"auto": sampler, "whole": sampler_whole, "split4": sampler_split}[request.param]
+
+
+@pytest.mark.parametrize("vocab", [1028, 4100, 32767, 32772, 65541, 151936])
+def test_options_and_sizes(ctx, vocab):
+    rng = np.random.default_rng(vocab)
+    stride = (vocab + 3) // 4 * 4
+    cfgs = [dict(temperature=t, topK=INF, topP=p, minP=m)
+            for t, p, m in [(1.0, 1.0, 0.05), (0.7, 0.9, 0.1), (1.5, 1.0, 0.004), (0.05, 1.0, 0.02),
+                            (1.0, 0.3, 0.01), (1.0, 1.0, 1.0), (1.0, 1.0, 2.0), (30.0, 0.5, 0.5),
+                            (1.0, 0.0, 0.05), (0.9, 0.95, 0.9)]]
+    rows = len(cfgs)
+    x = np.zeros((rows, stride), np.float32)
+    x[:, :vocab] = rng.standard_normal((rows, vocab)) * 2.5
+    for r in range(rows):
+        x[r, rng.integers(0, vocab, 8)] += 12.0
+    u = rng.random(rows)
+    u[0], u[1] = 0.0, 1.0 - 2.0 ** -53
+    hist = rng.integers(0, vocab, (rows, 40)).astype(np.int32)
+    cfgs[3]["repetitionPenalty"] = 1.3
+    cfgs[9].update(presencePenalty=0.4, frequencyPenalty=0.2)
+    _check(ctx, x, vocab, hist.reshape(-1), np.arange(rows + 1, dtype=np.int64) * 40, cfgs, u, 64,
+           f"min-p V={vocab}", want_cands=False)
+
+
+def test_unusual_rows(ctx):
+    """Masked rows, rows with no, one or two candidates, NaN, an infinite
+    maximum, a maximum that only the last logits hold, more candidates than
+    the list takes (finished by the general path), ties."""
+    rng = np.random.default_rng(3)
+    vocab, rows = 70002, 14
+    x = np.full((rows, 70004), -np.inf, np.float32)
+    base = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
+    x[1, 5] = -3.0                                   # one candidate
+    x[2, [7, 69999]] = [1.0, 0.5]                    # two, far apart
+    x[3, 40000:40050] = base[3, :50]                 # a grammar's few allowed ids
+    x[4, :vocab] = base[4]
+    x[4, ::3] = np.nan
+    x[5, :vocab] = base[5]
+    x[5, 123] = np.inf
+    x[6, 9] = np.inf                                 # infinite and alone
+    x[7, :vocab] = np.sort(base[7])                  # rises to the end
+    x[8, :vocab] = 0.25                              # all equal: every logit is a candidate
+    x[9, :vocab] = np.round(base[9])                 # ties among the candidates
+    x[10, :vocab] = base[10]
+    x[10, vocab - 1] = 60.0                          # the maximum past the last whole float4
+    x[11, :vocab] = base[11] - 3e38 * (rng.random(vocab) < 0.5)
+    x[12, :vocab] = -0.0
+    x[12, 10:20] = 0.0
+    x[13, :vocab] = base[13] * 1e-3                  # nearly flat: more than the list takes
+    cfgs = [dict(temperature=1.0, topK=INF, topP=1.0, minP=0.05, ) for _ in range(rows)]
+    cfgs[10]["temperature"] = 0.02
+    u = rng.random(rows)
+    _check(ctx, x, vocab, None, None, cfgs, u, 64, "min-p unusual rows", want_cands=False)
+
+
+def test_unaligned_rows_and_candidates_take_the_general_path(ctx):
+    rng = np.random.default_rng(4)
+    vocab, rows = 5003, 5
+    x = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)   # odd stride
+    cfgs = [dict(temperature=1.0, topK=INF, topP=0.95, minP=0.02)] * rows
+    u = rng.random(rows)
+    _check(ctx, x, vocab, None, None, cfgs, u, 64, "min-p unaligned", want_cands=False)
+    _check(ctx, x, vocab, None, None, cfgs, u, 64, "min-p candidates", want_cands=True)
+
+
+def test_mixed_batch(ctx):
+    """Min-p rows beside rows of every other route, twice (the counters are
+    back at zero)."""
+    rng = np.random.default_rng(6)
+    vocab, rows = 40000, 12
+    x = (rng.standard_normal((rows, vocab)) * 2.5).astype(np.float32)
+    kinds = [dict(topK=INF, minP=0.05), dict(topK=40), dict(topK=500), dict(topK=INF, topP=0.9),
+             dict(topK=3000, minP=0.1), dict(temperature=0.0)]
+    cfgs = [dict(kinds[r % 6], repetitionPenalty=1.1 if r % 2 else 1.0) for r in range(rows)]
+    hist = rng.integers(0, vocab, (rows, 30)).astype(np.int32)
+    for _ in range(2):
+        _check(ctx, x, vocab, hist.reshape(-1), np.arange(rows + 1, dtype=np.int64) * 30, cfgs,
+               rng.random(rows), 64, "min-p mixed", want_cands=False)
