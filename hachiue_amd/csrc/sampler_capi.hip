@@ -572,10 +572,9 @@ int sample_device(hs_context *ctx, float *d_logits, int32_t rows, int64_t row_st
   int rc = ensure_split(ctx, n_row, split, stream);
   if (rc) return rc;
   // so does the min-p kernel (whole rows where the general path takes them:
-  // unaligned ones and calls that want candidates)
-  const bool vec = (reinterpret_cast<uintptr_t>(d_logits) & 15u) == 0 && (row_stride & 3) == 0;
+  // calls that want candidates)
   const bool want_cands = d_cand_ids || d_cand_probs;
-  const int minp_split = vec && !want_cands ? choose_split(ctx, n_minp, vocab) : 1;
+  const int minp_split = !want_cands ? choose_split(ctx, n_minp, vocab) : 1;
   if (minp_split > 1) {
     const size_t parts = (size_t)n_minp * (size_t)minp_split;
     HS_HIP(ctx->minp_cand.ensure(parts * hs::kMinpHand * sizeof(unsigned long long)));
@@ -616,7 +615,7 @@ int sample_device(hs_context *ctx, float *d_logits, int32_t rows, int64_t row_st
   a.rows = rows;
   a.vocab = vocab;
   a.chunks = (int32_t)S;
-  a.vec = vec ? 1 : 0;
+  a.vec = ((reinterpret_cast<uintptr_t>(d_logits) & 15u) == 0 && (row_stride & 3) == 0) ? 1 : 0;
   a.want_cands = want_cands ? 1 : 0;
   a.n_pf = n_pf;
   a.n_row = n_row;

@@ -3518,7 +3518,7 @@ size_t large_smem_bytes() { return sizeof(LargeSmem); }
 // Per-row constants of the large path (wave-uniform).
 struct LargeRow {
   const float *rowp;
-  int V, vec;
+  int V;
   uint32_t T;      // 0: every finite logit is a candidate; else keys > T plus `tin` equal to T
   int tin, teq;    // candidates equal to T, logits equal to T
   uint32_t lo, hi; // key range of the candidates
@@ -3556,50 +3556,38 @@ __device__ __forceinline__ float large_pfast(const LargeRow &L, float v) {
   return (float)((double)(float)p * L.inv_S);
 }
 
-// Calls f(index, value) for every logit of the row.  Eight float4 (or, for
-// unaligned rows, eight logits) per thread are requested before any is used,
-// through a buffer resource: reads past the row return 0 and are skipped.
+// Calls f(index, value) for every logit of the row.  Seven float4 per thread
+// are requested before any is used, through a buffer resource: reads past the
+// row return 0 and are skipped.  (A 16-byte buffer read needs an address of 4
+// bytes only.  Rows that start elsewhere than at 16 bytes took one read per
+// logit here, and the general path instead of the two-pass and min-p kernels:
+// 64 x 151937, top-p without top-k, 199 us against 65 us now.)
 // The reads are cached (not non-temporal): the path makes several passes
 // over a row, and the rows the GPU holds at once (607 KB each at V = 151936)
 // fit the last-level cache, so the passes after the first are served there.
 template <typename F>
 __device__ __forceinline__ void large_pass(const LargeRow &L, F f) {
-  constexpr int U = 8;
+  constexpr int U = 7;
   const int tid = threadIdx.x;
-  if (L.vec) {
-    const int nfull = L.V >> 2;
-    const rsrc_t r4 = make_rsrc(L.rowp, 16u * (uint32_t)nfull);
-    for (int i0 = tid; i0 < nfull; i0 += U * kLT) {
-      f32x4 t[U];
+  const int nfull = L.V >> 2;
+  const rsrc_t r4 = make_rsrc(L.rowp, 16u * (uint32_t)nfull);
+  for (int i0 = tid; i0 < nfull; i0 += U * kLT) {
+    f32x4 t[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const auto x = __builtin_amdgcn_raw_buffer_load_b128(r4, (i0 + u * kLT) * 16, 0, 0);
-        t[u] = f32x4{__uint_as_float(x[0]), __uint_as_float(x[1]), __uint_as_float(x[2]),
-                     __uint_as_float(x[3])};
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int i = i0 + u * kLT;
-        if (i < nfull) {
-          f(4 * i, t[u][0]); f(4 * i + 1, t[u][1]); f(4 * i + 2, t[u][2]); f(4 * i + 3, t[u][3]);
-        }
-      }
+    for (int u = 0; u < U; ++u) {
+      const auto x = __builtin_amdgcn_raw_buffer_load_b128(r4, (i0 + u * kLT) * 16, 0, 0);
+      t[u] = f32x4{__uint_as_float(x[0]), __uint_as_float(x[1]), __uint_as_float(x[2]),
+                   __uint_as_float(x[3])};
     }
-    for (int e = 4 * nfull + tid; e < L.V; e += kLT) f(e, L.rowp[e]);
-  } else {
-    const rsrc_t r1 = make_rsrc(L.rowp, 4u * (uint32_t)L.V);
-    for (int e0 = tid; e0 < L.V; e0 += U * kLT) {
-      float t[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        t[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r1, (e0 + u * kLT) * 4, 0, 0));
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int e = e0 + u * kLT;
-        if (e < L.V) f(e, t[u]);
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u * kLT;
+      if (i < nfull) {
+        f(4 * i, t[u][0]); f(4 * i + 1, t[u][1]); f(4 * i + 2, t[u][2]); f(4 * i + 3, t[u][3]);
       }
     }
   }
+  for (int e = 4 * nfull + tid; e < L.V; e += kLT) f(e, L.rowp[e]);
 }
 
 __device__ __forceinline__ double wave_sum_f64(double x) {
@@ -4000,7 +3988,6 @@ __device__ __forceinline__ void large_row(const LaunchArgs &a, const RowPlan &P,
   LargeRow L;
   L.rowp = a.logits + (int64_t)row * a.stride;
   L.V = a.vocab;
-  L.vec = a.vec;
   L.T = 1u;       // every finite logit, for the first passes
   L.tin = L.teq = 0;
 
@@ -5572,13 +5559,12 @@ __device__ __forceinline__ bool large_fast(const LaunchArgs &a, const RowPlan &P
 }
 
 // Rows of lfast_list; a row it cannot finish is marked in large_retry for
-// large_kernel.  Unaligned rows and calls that want candidate outputs are
-// all handed back.  Four waves per SIMD: one workgroup per CU.
+// large_kernel.  Calls that want candidate outputs are all handed back.  Four waves per SIMD: one workgroup per CU.
 __global__ __launch_bounds__(kFT, 4) void large_fast_kernel(LaunchArgs a, Workspace ws) {
   extern __shared__ unsigned long long ldyn[];
   const int row = ws.lfast_list[blockIdx.x];
   const RowPlan P = ws.plans[row];
-  const bool ok = a.vec && !a.want_cands && a.vocab < (1 << 26) &&
+  const bool ok = !a.want_cands && a.vocab < (1 << 26) &&
                   large_fast(a, P, row, *reinterpret_cast<FastSmem *>(ldyn));
   if (threadIdx.x == 0) ws.large_retry[blockIdx.x] = ok ? 0 : 1;
 }
@@ -5626,7 +5612,7 @@ __global__ __launch_bounds__(kLT) void large_kernel(LaunchArgs a, Workspace ws) 
 //    top-p stops and the draw from it (src/sampler.ts:83-117).
 // A row this does not suit (more than kMpCap logits listed by a part or
 // kSortCap kept, an infinite maximum, a normaliser that is not finite,
-// unaligned rows, candidate outputs) is finished by large_row instead, by the
+// candidate outputs) is finished by large_row instead, by the
 // same workgroup.
 // Bound: one read of the row; the general path reads it four to six times
 // with one workgroup per row.  50 rows x 151936, min-p 0.05, repetition 1.1:
@@ -5928,12 +5914,16 @@ __global__ __launch_bounds__(kRowThreads) void minp_kernel(LaunchArgs a, Workspa
   extern __shared__ unsigned long long ldyn[];
   __shared__ ReplayReq unused_req;   // k = vocab: never a replay
   const int slot = (int)blockIdx.x / a.minp_split, part = (int)blockIdx.x - slot * a.minp_split;
-  const int row = ws.minp_list[slot];
-  const RowPlan P = ws.plans[row];
-  if (a.vec && !a.want_cands) {   // (otherwise minp_split is 1)
-    if (minp_row(a, ws, P, row, slot, part, *reinterpret_cast<MinpSmem *>(ldyn))) return;
+  if (!a.want_cands) {   // (otherwise minp_split is 1)
+    const int row = ws.minp_list[slot];
+    if (minp_row(a, ws, ws.plans[row], row, slot, part, *reinterpret_cast<MinpSmem *>(ldyn))) return;
     __syncthreads();   // (uniform: the LDS is large_row's from here)
   }
+  // (the plan is read again: kept from above it would cost registers, spilled)
+  int again = slot;
+  asm volatile("" : "+s"(again));
+  const int row = ws.minp_list[again];
+  const RowPlan P = ws.plans[row];
   large_row(a, P, row, *reinterpret_cast<LargeSmem *>(ldyn), &unused_req);
 }
 

@@ -70,14 +70,19 @@ def test_unusual_rows(ctx):
     _check(ctx, x, vocab, None, None, cfgs, u, 64, "min-p unusual rows", want_cands=False)
 
 
-def test_unaligned_rows_and_candidates_take_the_general_path(ctx):
-    rng = np.random.default_rng(4)
-    vocab, rows = 5003, 5
-    x = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)   # odd stride
-    cfgs = [dict(temperature=1.0, topK=INF, topP=0.95, minP=0.02)] * rows
+@pytest.mark.parametrize("vocab", [1025, 5003, 65538, 151939])
+@pytest.mark.parametrize("opts", [dict(minP=0.02), dict(), dict(topK=3000, minP=0.02)])
+def test_unaligned_rows(ctx, vocab, opts):
+    """Odd strides: rows that start at any multiple of four bytes, on the
+    min-p, two-pass and general kernels; then with candidate outputs (the
+    general path)."""
+    rng = np.random.default_rng(vocab)
+    rows = 5
+    x = (rng.standard_normal((rows, vocab)) * 2).astype(np.float32)
+    cfgs = [dict(dict(temperature=1.0, topK=INF, topP=0.95), **opts)] * rows
     u = rng.random(rows)
-    _check(ctx, x, vocab, None, None, cfgs, u, 64, "min-p unaligned", want_cands=False)
-    _check(ctx, x, vocab, None, None, cfgs, u, 64, "min-p candidates", want_cands=True)
+    _check(ctx, x, vocab, None, None, cfgs, u, 64, "unaligned", want_cands=False)
+    _check(ctx, x, vocab, None, None, cfgs, u, 64, "unaligned, candidates", want_cands=True)
 
 
 def test_mixed_batch(ctx):
