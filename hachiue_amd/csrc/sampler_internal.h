@@ -276,12 +276,24 @@ constexpr int gemv_lds_bytes(int type) { return (kGemvThreads / 64) * gemv_batch
 hipError_t launch_gemv(const GemvArgs &g, hipStream_t stream, hipEvent_t *ev, hipEvent_t done);
 hipError_t prepare_gemv();      // per device, once (called by prepare_kernels)
 // Several activation rows in one pass over the weights (batch_gemv.hip), the
-// rows of one launch, and the bytes of their limb tables (16 slices of 16
-// rows, K / 256 blocks of at most 17152 bytes each).
+// rows of one launch, and the bytes of their tables (16 slices of 16 rows,
+// K / 256 blocks of at most 17408 bytes each).
 constexpr int kBatchRows = 256;
-constexpr size_t kBatchTabBytes = (size_t)(kBatchRows / 16) * (kGemvMaxK / 256) * 17152;
-constexpr bool gemv_batched(int type, int M) {
-  return M >= 2 && (type == kW_Q6_K || type == kW_Q4_K);
+constexpr size_t kBatchTabBytes = (size_t)(kBatchRows / 16) * (kGemvMaxK / 256) * 17408;
+// From which M on: the K-quants, Q1_0 and PQ2_0 at once (2 rows 70 against 96
+// us, 22 against 29, 23 against 34); PTQ1_0 from 3 (2 rows take 42 us either
+// way, and greedy calls would lose their one launch); the others from 4 (one
+// row at a time their greedy calls may run in one launch, whose sums are the
+// GEMV's bit for bit).
+constexpr bool gemv_batched(int type, int M, int K) {
+  switch (type) {
+    case kW_Q6_K: case kW_Q4_K: return M >= 2;
+    case kW_Q1_0: case kW_PQ2_0: return M >= 2 && K % 512 == 0;
+    case kW_PTQ1_0: return M >= 3 && K % 512 == 0;
+    case kW_Q4_0: case kW_Q4_1: return M >= 4 && K % 256 == 0;
+    case kW_F32: return M >= 4 && K % 64 == 0;
+    default: return false;
+  }
 }
 hipError_t launch_gemv_batch(GemvArgs g, hipStream_t stream, hipEvent_t *ev, hipEvent_t done);
 hipError_t prepare_gemv_batch();   // per device, once (called by prepare_gemv)

@@ -5,56 +5,65 @@ one of tests/test_gpu_lmhead.py, 2^-16 sum_k |x_k w_k| per logit."""
 import numpy as np
 import pytest
 
-from hachiue_amd import hip
-from oracle import pyoracle as o
-from tests.test_gpu_lmhead import FORMATS, check, run_gemv
+from tests.test_gpu_lmhead import FORMATS, PLANAR, check, run_gemv, run_gemv_ex
 from tests.test_oracle_lmhead import random_blocks
 
 pytestmark = pytest.mark.gpu
 
-BATCHED = ["q4_k", "q6_k"]
+ALL = dict(FORMATS, **PLANAR)
+STEP = {"f32": 64, "q4_0": 256, "q4_1": 256, "q4_k": 256, "q6_k": 256}   # of K; planar 512
 
 
-@pytest.mark.parametrize("fmt", BATCHED)
-@pytest.mark.parametrize("M,K,N", [(2, 256, 16), (3, 512, 33), (4, 4096, 1000), (5, 256, 4099),
-                                   (8, 1024, 17), (9, 768, 5000), (16, 512, 65), (17, 256, 4096),
-                                   (32, 4096, 200), (33, 512, 999), (64, 1024, 3001),
-                                   (259, 512, 40)])
+def run(sampler, fmt, x, w, N, pad=0):
+    if fmt in PLANAR:
+        return run_gemv_ex(sampler, ALL[fmt], x, w, N, ldx=x.shape[1] + pad, ldy=N + pad)
+    return run_gemv(sampler, ALL[fmt], x, w, N, ldx=x.shape[1] + pad, ldy=N + pad)
+
+
+@pytest.mark.parametrize("fmt", list(ALL))
+@pytest.mark.parametrize("M,K,N", [(2, 1, 16), (3, 2, 33), (4, 0, 1000), (5, 1, 4099),
+                                   (8, 4, 17), (9, 3, 5000), (16, 2, 65), (17, 1, 4096),
+                                   (32, 0, 200), (33, 2, 999), (64, 3, 3001), (259, 1, 40)])
 def test_batched_rows(sampler, fmt, M, K, N):
+    """K in steps of the format's slab (0: the longest, 4096)."""
+    K = K * STEP.get(fmt, 512) or 4096
     rng = np.random.default_rng(M * 1000 + K + N)
-    w = random_blocks(FORMATS[fmt], N, K, rng)
+    w = random_blocks(ALL[fmt], N, K, rng)
     x = rng.standard_normal((M, K)).astype(np.float32)
     x[M // 2] *= np.exp2(rng.integers(-20, 20, K)).astype(np.float32)
     x[-1, ::3] = 0.0
-    y = run_gemv(sampler, FORMATS[fmt], x, w, N, ldx=K + 4, ldy=N + 3)
-    check(FORMATS[fmt], x, w, N, y)
+    y = run(sampler, fmt, x, w, N, pad=3)
+    check(ALL[fmt], x, w, N, y)
 
 
-@pytest.mark.parametrize("fmt", BATCHED)
+@pytest.mark.parametrize("fmt", list(ALL))
 def test_batched_rows_full_vocabulary(sampler, fmt):
     rng = np.random.default_rng(5)
-    M, K, N = 20, 1024, 151936
-    w = random_blocks(FORMATS[fmt], N, K, rng)
+    M, K, N = 20, 512 if fmt == "f32" else 1024, 151936
+    w = random_blocks(ALL[fmt], N, K, rng)
     x = rng.standard_normal((M, K)).astype(np.float32)
-    y = run_gemv(sampler, FORMATS[fmt], x, w, N)
-    check(FORMATS[fmt], x[[0, 7, 19]], w, N, y[[0, 7, 19]])
-    # the same rows again, alone in their slice: a row's logits do not depend
-    # on its neighbours
-    again = run_gemv(sampler, FORMATS[fmt], x[17:], w, N)
-    check(FORMATS[fmt], x[[19]], w, N, again[[2]])
+    y = run(sampler, fmt, x, w, N)
+    check(ALL[fmt], x[[0, 7, 19]], w, N, y[[0, 7, 19]])
+    # some of the rows again, in a smaller batch
+    again = run(sampler, fmt, x[13:], w, N)
+    check(ALL[fmt], x[[19]], w, N, again[[6]])
 
 
-@pytest.mark.parametrize("fmt", ["q4_k", "q6_k"])
+@pytest.mark.parametrize("fmt", list(ALL))
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
 def test_batched_row_with_non_finite_input(sampler, fmt, bad):
-    """The row of a non-finite element is NaN everywhere, its neighbours are
+    """The row of a non-finite element has no finite logit where its weight
+    is not 0, and is NaN everywhere on the integer formats; its neighbours are
     untouched."""
     rng = np.random.default_rng(9)
     M, K, N = 11, 512, 300
-    w = random_blocks(FORMATS[fmt], N, K, rng)
+    w = random_blocks(ALL[fmt], N, K, rng)
     x = rng.standard_normal((M, K)).astype(np.float32)
     x[6, 300] = bad
-    y = run_gemv(sampler, FORMATS[fmt], x, w, N)
-    assert np.isnan(y[6]).all()
+    y = run(sampler, fmt, x, w, N)
+    if fmt in ("f32", "q4_0", "q4_1"):
+        assert not np.isfinite(y[6]).any()
+    else:
+        assert np.isnan(y[6]).all()
     keep = [r for r in range(M) if r != 6]
-    check(FORMATS[fmt], x[keep], w, N, y[keep])
+    check(ALL[fmt], x[keep], w, N, y[keep])
