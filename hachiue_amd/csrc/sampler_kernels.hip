@@ -1290,6 +1290,8 @@ struct RowScratch {          // LDS arrays of at least k entries each
   double *sp;
   float *rsv;
   int32_t *rsid;
+  unsigned long long *big;     // LDS for the slot chains (the arrays above and srt lie in
+  int big_words;               //   it): 64-bit words, then a ChaseSmem
 };
 
 // atomicMin(dst, i) for the first lane of the wave whose pred holds, i rising
@@ -1404,6 +1406,162 @@ __device__ __forceinline__ void tail_block(int n, const RowPlan &P, double u, Ro
   __syncthreads();
 }
 
+// ---- equal values of a mid row, by the chains of their slots
+//
+// A draw inside a group of equal logits needs the members' order by slot
+// (src/sampler.ts:50-74).  The whole scan is not needed for that: a logit that
+// enters at index i takes the slot of the logit that leaves, the smallest of
+// the k largest of [0, i), and that one entered earlier, so a member's slot
+// is found by going back from logit to logit until one of the first k, whose
+// slot is its index: about ln(V / k) steps on random rows.  All of it runs on
+// a list of the logits that can ever have been in a slot: the first k, then of
+// each stretch [P, r P) those above the k-th largest of [0, P) (about k (r -
+// 1) of them), which the next stretch's bound is selected from.
+// Not settled here (-1; the scan is replayed): a leaving value that the list
+// holds twice in the prefix (the smallest slot of several would leave), a row
+// whose first k logits are not all finite, more than kChaseMembers members or
+// kChaseSteps steps, a list that does not fit.
+// 256 x 151936, one row with such a draw (about one in 10,000 rows of k <=
+// 1024 on random logits has one): 205 us a call at k 1000, 161 at k 300 (58
+// and 39 without the draw); with the scan 8824 and 2039.  The state lies in
+// the tail's LDS: static LDS of its own moved the stream's arrays and cost the
+// kernel 1.5 %.
+constexpr int kChaseMembers = 16;
+constexpr int kChaseSteps = 64;
+constexpr int kChaseHist = 2048;   // words of the select's histogram
+struct ChaseSmem {
+  uint32_t wsum[16];
+  int32_t n, dig, rem, cnt, idx;
+  int32_t mem[kChaseMembers], slot[kChaseMembers];
+  int32_t pad;
+};
+
+// The k-th largest key among the list's entries (key << 32 | index) of index
+// below lim, by three digit passes; 0 when there are fewer than k.  With
+// `who`, c.cnt counts those of that key and c.idx is (one of) their indices.
+template <int NT>
+__device__ __forceinline__ uint32_t chase_kth(const unsigned long long *list, int n, uint32_t lim, int k,
+                                              bool who, uint32_t *hist, ChaseSmem &c) {
+  const int tid = threadIdx.x;
+  uint32_t prefix = 0;
+  int rem = k;
+#pragma nounroll
+  for (int pass = 0; pass < 3; ++pass) {
+    const int sh = pass == 0 ? 21 : pass == 1 ? 10 : 0, nd = pass == 2 ? 1024 : 2048;
+    const int top = pass == 0 ? 31 : sh + (pass == 1 ? 11 : 10);
+    for (int i = tid; i < kChaseHist; i += NT) hist[i] = 0u;
+    if (tid == 0) c.dig = -1;
+    __syncthreads();
+    for (int i = tid; i < n; i += NT) {
+      const unsigned long long e = list[i];
+      const uint32_t key = (uint32_t)(e >> 32);
+      if ((uint32_t)e < lim && (pass == 0 || (key >> top) == (prefix >> top)))
+        atomicAdd(&hist[(key >> sh) & (uint32_t)(nd - 1)], 1u);
+    }
+    __syncthreads();
+    // thread t owns digits nd - 1 - 2t and nd - 2 - 2t (descending)
+    const int d = nd - 1 - 2 * tid;
+    const uint32_t c0 = d > 0 ? hist[d] : 0u, c1 = d > 0 ? hist[d - 1] : 0u;
+    const uint32_t ex = block_scan_incl<NT>(c0 + c1, c.wsum) - (c0 + c1);   // one barrier inside
+    if (ex < (uint32_t)rem && ex + c0 + c1 >= (uint32_t)rem) {
+      const bool first = ex + c0 >= (uint32_t)rem;
+      c.dig = first ? d : d - 1;
+      c.rem = rem - (int)(first ? ex : ex + c0);
+    }
+    __syncthreads();
+    if (c.dig < 0) return 0u;   // (uniform)
+    prefix |= (uint32_t)c.dig << sh;
+    rem = c.rem;
+    __syncthreads();
+  }
+  if (who) {
+    if (tid == 0) c.cnt = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += NT) {
+      const unsigned long long e = list[i];
+      if ((uint32_t)e < lim && (uint32_t)(e >> 32) == prefix) {
+        atomicAdd(&c.cnt, 1);
+        c.idx = (int32_t)(uint32_t)e;
+      }
+    }
+    __syncthreads();
+  }
+  return prefix;
+}
+
+// The index of the rank-th of the g group members c.mem (indices) in slot
+// order, or -1.  buf: `words` 64-bit words of LDS for the list and the
+// histogram.
+template <int NT>
+__device__ __forceinline__ int chase_pick(const float *rowp, int V, int k, int g, int rank,
+                                          unsigned long long *buf, int words, ChaseSmem &c) {
+  // (nothing of this rare path is computed ahead of it: the row's stream
+  // has no registers to spare)
+  asm volatile("" : "+s"(V), "+s"(k), "+s"(rowp));
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int cap = words - kChaseHist / 2;
+  unsigned long long *list = buf;
+  uint32_t *hist = reinterpret_cast<uint32_t *>(buf + cap);
+  if (g > kChaseMembers || k >= V || k > cap) return -1;
+  int bad = 0;
+  for (int i = tid; i < k; i += NT) {
+    const uint32_t key = f2key(rowp[i]);
+    bad |= key == 0u;
+    list[i] = ((unsigned long long)key << 32) | (uint32_t)i;
+  }
+  if (tid == 0) c.n = k;
+  if (__syncthreads_or(bad)) return -1;
+  // stretches of four times the prefix while the list then fits, else of two
+  int p4 = 0;
+  for (int p = k; p < V && p <= (1 << 28); p *= 4) ++p4;
+  const int ratio = k * (1 + 3 * p4) <= cap ? 4 : 2;
+  for (int64_t P = k; P < V; P *= ratio) {
+    const uint32_t th = chase_kth<NT>(list, c.n, 0xFFFFFFFFu, k, false, hist, c);
+    const int Q = (int)(P * ratio < V ? P * ratio : V);
+    for (int e0 = (int)P; e0 < Q; e0 += 4 * NT) {
+      float x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int e = e0 + u * NT + tid;
+        x[u] = rowp[e < Q ? e : 0];   // always a read inside the row
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int e = e0 + u * NT + tid;
+        const uint32_t key = e < Q ? f2key(x[u]) : 0u;
+        const unsigned long long m = __ballot(key > th);
+        if (m == 0ull) continue;
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&c.n, __popcll(m));
+        base = __builtin_amdgcn_readfirstlane(base);
+        const int p = base + (int)lanes_below(m);
+        if (key > th && p < cap) list[p] = ((unsigned long long)key << 32) | (uint32_t)e;
+      }
+    }
+    __syncthreads();
+    if (c.n > cap) return -1;
+  }
+  const int n = c.n;
+  for (int i = 0; i < g; ++i) {
+    int cur = c.mem[i];
+    for (int step = 0; cur >= k; ++step) {
+      if (step == kChaseSteps || chase_kth<NT>(list, n, (uint32_t)cur, k, true, hist, c) == 0u || c.cnt != 1)
+        return -1;   // (uniform)
+      cur = c.idx;
+      __syncthreads();
+    }
+    if (tid == 0) c.slot[i] = cur;
+  }
+  __syncthreads();
+  // (slots are distinct)
+  for (int i = 0; i < g; ++i) {
+    int below = 0;
+    for (int j = 0; j < g; ++j) below += c.slot[j] < c.slot[i];
+    if (below == rank) return c.mem[i];
+  }
+  return -1;
+}
+
 // Completes a top-k row.  `srt` holds n_sel packed candidates, every logit
 // with key >= T (the exact k-th largest key; all candidates when fewer than
 // k), sorted descending.  closed_form: no slot was ever evicted (at most k
@@ -1437,10 +1595,14 @@ __device__ __forceinline__ void finish_row(const LaunchArgs &a, const RowPlan &P
   __syncthreads();
 
   // tail, src/sampler.ts:76-117; runs twice when a tie group holds the draw
+  // and the members' slots are not settled by their chains
   const double u = a.uniforms[row];
+  int chased = -1;   // the token by the slot chains
   for (int attempt = 0; attempt < 2; ++attempt) {
     if (need_replay) {
-      if (tid < 64) replay_row<NT == kRowThreads ? 8 : 32>(rowp, a.vocab, k, s.rsv, s.rsid);
+      // (4 blocks ahead: 8 and the slot chains' code together cost the rows
+      // without a replay 0.6 %)
+      if (tid < 64) replay_row<NT == kRowThreads ? 4 : 32>(rowp, a.vocab, k, s.rsv, s.rsid);
       __syncthreads();
       if (tid == 0) f.n_sel = 0;
       __syncthreads();
@@ -1478,6 +1640,26 @@ __device__ __forceinline__ void finish_row(const LaunchArgs &a, const RowPlan &P
         const uint32_t kp = s.skey[pick];
         hit = (pick > 0 && s.skey[pick - 1] == kp) || (pick + 1 < n && s.skey[pick + 1] == kp) ||
               (boundary_tie && kp == T);
+        if constexpr (NT == kRowThreads) {
+          // every logit of the drawn value is a candidate: their slots alone
+          // are needed
+          if (__builtin_expect(hit && !(boundary_tie && kp == T), 0)) {
+            ChaseSmem &cs = *reinterpret_cast<ChaseSmem *>(s.big + s.big_words);
+            int lo = pick, hi = pick + 1;
+            while (lo > 0 && pick - lo < kChaseMembers && s.skey[lo - 1] == kp) --lo;
+            while (hi < n && hi - pick < kChaseMembers && s.skey[hi] == kp) ++hi;
+            const int g = hi - lo;
+            if (tid < g && tid < kChaseMembers) cs.mem[tid] = s.sids[lo + tid];
+            __syncthreads();   // (the arrays are the list's from here)
+            chased = chase_pick<NT>(rowp, a.vocab, k, g, pick - lo, s.big, s.big_words, cs);
+            __syncthreads();
+            if (chased >= 0) {
+              if (tid == 0) f.replay = 1;
+              __syncthreads();
+              break;
+            }
+          }
+        }
       }
       if (hit) { need_replay = true; continue; }
     }
@@ -1487,7 +1669,7 @@ __device__ __forceinline__ void finish_row(const LaunchArgs &a, const RowPlan &P
   const int cs = a.cand_stride;
   if (tid == 0) {
     const int pick = f.pick;
-    put_token(a, row, pick >= 0 ? s.sids[pick] : 0);
+    put_token(a, row, chased >= 0 ? chased : pick >= 0 ? s.sids[pick] : 0);
     if (a.cand_count_out) a.cand_count_out[row] = n;
     if (a.cutoff_out) a.cutoff_out[row] = f.cutoff;
     if (a.row_flags) {
@@ -3212,6 +3394,10 @@ __global__ __launch_bounds__(kRowThreads) void mid_kernel(LaunchArgs a, Workspac
   sc.sp = reinterpret_cast<double *>(hist + 3 * kMaxK);
   sc.rsv = reinterpret_cast<float *>(hist + 5 * kMaxK);
   sc.rsid = reinterpret_cast<int32_t *>(hist + 6 * kMaxK);
+  sc.big = cbuf;   // cbuf, srt and hist
+  sc.big_words = kRowCandCap + kSortCap + kMidBins / 2 - (int)(sizeof(ChaseSmem) / 8);
+  static_assert(sizeof(ChaseSmem) % 8 == 0 && 7 * kMaxK * 4 + sizeof(ChaseSmem) <= kMidBins * 4,
+                "the chains' state past the tail's arrays");
   // closed form: all finite logits are candidates and there are at most k
   finish_row<kRowThreads>(a, P, row, rowp, srt, n_sel, T, theta == 0 && n <= k, overflow, sc,
                           ms.tail);
