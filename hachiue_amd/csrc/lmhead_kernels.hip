@@ -76,11 +76,11 @@ __global__ __launch_bounds__(KqBody<FMT>::kThreads, 2) void gemv_kq_mfma_kernel(
 
 
 
-template <int FMT>
+template <int FMT, bool ROT>
 __global__ __launch_bounds__(64 * tm::waves<FMT>()) void gemv_tern_kernel(GemvArgs g) {
   extern __shared__ uint4 tlds[];
   StoreRow epi{g.y + (int64_t)blockIdx.y * g.ldy};
-  tern_gemv_body<FMT>(g, tlds, epi);
+  tern_gemv_body<FMT, ROT>(g, tlds, epi);
 }
 
 // ---- the 512-wide Hadamard rotation (src/kernels.ts:177-227, mode 0)
@@ -197,21 +197,21 @@ hipError_t launch_kq_mfma(GemvArgs g, hipStream_t stream, hipEvent_t *ev, hipEve
   return hipGetLastError();
 }
 
-template <int FMT>
+template <int FMT, bool ROT>
 hipError_t launch_tern(GemvArgs g, hipStream_t stream, hipEvent_t *ev, hipEvent_t done) {
   const size_t lds = gemv_tern_lds_bytes(g.K);
   const int ntiles = (g.N + 15) / 16;
   // one workgroup per CU (its LDS holds two out), at most one per tile
-  const int res = resident_blocks(reinterpret_cast<const void *>(gemv_tern_kernel<FMT>),
+  const int res = resident_blocks(reinterpret_cast<const void *>(gemv_tern_kernel<FMT, ROT>),
                                   (uint32_t)lds, 64 * tm::waves<FMT>());
   const int blocks = ntiles < res ? ntiles : res;
   const dim3 grid((unsigned)blocks, (unsigned)g.M), block(64 * tm::waves<FMT>());
   if (ev)
-    hipExtLaunchKernelGGL(gemv_tern_kernel<FMT>, grid, block, lds, stream, ev[0], ev[1], 0u, g);
+    hipExtLaunchKernelGGL((gemv_tern_kernel<FMT, ROT>), grid, block, lds, stream, ev[0], ev[1], 0u, g);
   else if (done)
-    hipExtLaunchKernelGGL(gemv_tern_kernel<FMT>, grid, block, lds, stream, nullptr, done, 0u, g);
+    hipExtLaunchKernelGGL((gemv_tern_kernel<FMT, ROT>), grid, block, lds, stream, nullptr, done, 0u, g);
   else
-    hipLaunchKernelGGL(gemv_tern_kernel<FMT>, grid, block, lds, stream, g);
+    hipLaunchKernelGGL((gemv_tern_kernel<FMT, ROT>), grid, block, lds, stream, g);
   return hipGetLastError();
 }
 
@@ -227,9 +227,12 @@ hipError_t prepare_gemv() {
     e = hipFuncSetAttribute(reinterpret_cast<const void *>(gemv_kq_mfma_kernel<kW_Q4_K>),
                             hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)KqBody<kW_Q4_K>::lds(kGemvMaxK));
-  const void *tk[3] = {reinterpret_cast<const void *>(gemv_tern_kernel<kW_Q1_0>),
-                       reinterpret_cast<const void *>(gemv_tern_kernel<kW_PQ2_0>),
-                       reinterpret_cast<const void *>(gemv_tern_kernel<kW_PTQ1_0>)};
+  const void *tk[6] = {reinterpret_cast<const void *>(gemv_tern_kernel<kW_Q1_0, false>),
+                       reinterpret_cast<const void *>(gemv_tern_kernel<kW_PQ2_0, false>),
+                       reinterpret_cast<const void *>(gemv_tern_kernel<kW_PTQ1_0, false>),
+                       reinterpret_cast<const void *>(gemv_tern_kernel<kW_Q1_0, true>),
+                       reinterpret_cast<const void *>(gemv_tern_kernel<kW_PQ2_0, true>),
+                       reinterpret_cast<const void *>(gemv_tern_kernel<kW_PTQ1_0, true>)};
   for (const void *f : tk)
     if (e == hipSuccess)
       e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -254,9 +257,12 @@ hipError_t launch_gemv(const GemvArgs &g, hipStream_t stream, hipEvent_t *ev, hi
     case kW_Q4_1: return two ? launch_fmt<kW_Q4_1, 2>(g, stream, ev, done) : launch_fmt<kW_Q4_1, 1>(g, stream, ev, done);
     case kW_Q4_K: return launch_kq_mfma<kW_Q4_K>(g, stream, ev, done);
     case kW_Q6_K: return launch_kq_mfma<kW_Q6_K>(g, stream, ev, done);
-    case kW_Q1_0: return launch_tern<kW_Q1_0>(g, stream, ev, done);
-    case kW_PQ2_0: return launch_tern<kW_PQ2_0>(g, stream, ev, done);
-    case kW_PTQ1_0: return launch_tern<kW_PTQ1_0>(g, stream, ev, done);
+    case kW_Q1_0: return g.rotate ? launch_tern<kW_Q1_0, true>(g, stream, ev, done)
+                                  : launch_tern<kW_Q1_0, false>(g, stream, ev, done);
+    case kW_PQ2_0: return g.rotate ? launch_tern<kW_PQ2_0, true>(g, stream, ev, done)
+                                  : launch_tern<kW_PQ2_0, false>(g, stream, ev, done);
+    case kW_PTQ1_0: return g.rotate ? launch_tern<kW_PTQ1_0, true>(g, stream, ev, done)
+                                  : launch_tern<kW_PTQ1_0, false>(g, stream, ev, done);
     default: return hipErrorInvalidValue;
   }
 }

@@ -186,7 +186,7 @@ struct hs_context {
   DevBuf plans, cand, cand_count, info;
   DevBuf split_list, split_meta, split_cnt;   // split rows (split_cnt: zero between calls)
   DevBuf gemv_part, gemv_cnt;   // Q4_K/Q6_K GEMV tiles cut between waves (gemv_cnt: zero between calls)
-  DevBuf gemv_rot;              // the Hadamard-rotated input of a folded weight
+  DevBuf gemv_rot;              // the Hadamard-rotated input of a folded weight (see gemv_setup)
   DevBuf gemv_tab;              // limb tables of several activation rows (one size, for good)
   DevBuf fuse_rows, fuse_pool, fuse_hist;   // lm_head GEMV that samples its rows: counters
                                 //   (zero between calls), the waves' two largest, the
@@ -710,7 +710,8 @@ int argmax_device(hs_context *ctx, const float *d_logits, int32_t rows, int64_t 
 // src/engine.ts:1493-1515 (the lm_head GEMV; see lmhead_kernels.hip).
 // The checks and arguments of an lm_head GEMV call, on the call's stream
 // (entered: enter_stream ran).  A Hadamard-folded weight's input is rotated
-// here, into the workspace.  *skip: nothing to compute (M or N is 0).
+// here, into the workspace, except where the GEMV does it (planar formats, a
+// row at a time).  *skip: nothing to compute (M or N is 0).
 int gemv_setup(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, const hs_weights *wt,
                float *d_y, int64_t ldy, hipStream_t stream, hs::GemvArgs &g, bool *skip) {
   *skip = false;
@@ -806,7 +807,10 @@ int gemv_setup(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, const 
     g.part = static_cast<float *>(ctx->gemv_part.p);
     g.tile_cnt = static_cast<uint32_t *>(ctx->gemv_cnt.p);
   }
-  if (wt->hadamard) {   // src/engine.ts:1121-1145: the input is rotated first
+  if (wt->hadamard && planar && !g.tab) {   // rotated by the GEMV itself
+    g.rotate = 1;
+    g.signs = wt->signs;
+  } else if (wt->hadamard) {   // src/engine.ts:1121-1145: the input is rotated first
     HS_HIP(ctx->gemv_rot.ensure((size_t)M * (size_t)K * sizeof(float)));
     float *rot = static_cast<float *>(ctx->gemv_rot.p);
     const hipError_t e = hs::launch_hadamard(d_x, ldx, wt->signs, rot, M, K, stream);

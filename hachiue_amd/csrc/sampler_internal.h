@@ -252,6 +252,10 @@ struct GemvArgs {
   // block scales (N * K / 128 of each), s_bytes their size
   const void *scales;
   uint32_t s_bytes;
+  // and, for a Hadamard-folded weight, that x is to be rotated first, with
+  // these signs (or null): the kernel does it (the others' x comes rotated)
+  int32_t rotate;
+  const float *signs;
   // several activation rows in one pass over the weights (batch_gemv.hip):
   // the workspace of their limb tables, or null for a row at a time
   void *tab;

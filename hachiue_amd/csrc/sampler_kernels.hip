@@ -6583,7 +6583,7 @@ __device__ void fuse_sample_finish(const GemvArgs &g, const FuseArgs &f, int m, 
 }
 
 // (one 16-wave workgroup per CU, as the plain GEMV)
-template <int FMT>
+template <int FMT, bool ROT>
 __global__ __launch_bounds__(64 * tm::waves<FMT>()) void gemv_tern_sample_kernel(GemvArgs g,
                                                                                    FuseArgs f) {
   constexpr int NW = tm::waves<FMT>();
@@ -6603,7 +6603,7 @@ __global__ __launch_bounds__(64 * tm::waves<FMT>()) void gemv_tern_sample_kernel
   uint8_t *lb = reinterpret_cast<uint8_t *>(tlds);
   uint2 *rec = reinterpret_cast<uint2 *>(lb + gemv_tern_lds_bytes(g.K));
   RecordEpi epi{y, rec + wave * kFuseTiles * 16, rep ? fs.rset : nullptr, 0, kFuseTiles};
-  tern_gemv_body<FMT>(g, tlds, epi);
+  tern_gemv_body<FMT, ROT>(g, tlds, epi);
   int32_t *more = reinterpret_cast<int32_t *>(rec + NW * kFuseTiles * 16);
   fuse_sample_finish<NW>(g, f, m, epi.nt, kFuseTiles, rec, more,
                          reinterpret_cast<unsigned long long *>(more + kFuseMore), fs);
@@ -6616,7 +6616,8 @@ template <int FMT>
 int tern_sample_blocks(const GemvArgs &g, size_t lds) {
   constexpr int nw = tm::waves<FMT>();
   const int ntiles = (g.N + 15) / 16;
-  const int res = resident_blocks(reinterpret_cast<const void *>(gemv_tern_sample_kernel<FMT>),
+  const int res = resident_blocks(g.rotate ? reinterpret_cast<const void *>(gemv_tern_sample_kernel<FMT, true>)
+                                           : reinterpret_cast<const void *>(gemv_tern_sample_kernel<FMT, false>),
                                   (uint32_t)lds, 64 * nw);
   const int blocks = ntiles < res ? ntiles : res;
   return tern_out_tiles_max(g.N, g.K, blocks, nw) <= kFuseTiles &&
@@ -6700,7 +6701,7 @@ __device__ __forceinline__ void fuse_argmax_finish(const GemvArgs &g, const Fuse
   }
 }
 
-template <int FMT>
+template <int FMT, bool ROT>
 __global__ __launch_bounds__(64 * tm::waves<FMT>())
 void gemv_tern_argmax_kernel(GemvArgs g, FuseArgs f) {
   constexpr int NW = tm::waves<FMT>();
@@ -6716,7 +6717,7 @@ void gemv_tern_argmax_kernel(GemvArgs g, FuseArgs f) {
   if (rep) fuse_rep_set(f, m, g.N, rset);
   // (the body's first barrier completes the set)
   ArgmaxEpi epi{g.y + (int64_t)m * g.ldy, rep ? rset : nullptr, load_scalar(&plan->rep), 0ull};
-  tern_gemv_body<FMT>(g, tlds, epi);
+  tern_gemv_body<FMT, ROT>(g, tlds, epi);
   fuse_argmax_finish<NW>(g, f, m, epi.best, wbest);
 }
 
@@ -6855,9 +6856,13 @@ int argmax_fused_grid(const GemvArgs &g) {
   }
   const int nw = g.type == kW_Q1_0 ? tm::waves<kW_Q1_0>()
                  : g.type == kW_PQ2_0 ? tm::waves<kW_PQ2_0>() : tm::waves<kW_PTQ1_0>();
-  const void *k = g.type == kW_Q1_0 ? reinterpret_cast<const void *>(gemv_tern_argmax_kernel<kW_Q1_0>)
-                  : g.type == kW_PQ2_0 ? reinterpret_cast<const void *>(gemv_tern_argmax_kernel<kW_PQ2_0>)
-                                       : reinterpret_cast<const void *>(gemv_tern_argmax_kernel<kW_PTQ1_0>);
+  auto pick = [&](auto plain, auto rotating) {
+    return g.rotate ? reinterpret_cast<const void *>(rotating) : reinterpret_cast<const void *>(plain);
+  };
+  const void *k = g.type == kW_Q1_0 ? pick(gemv_tern_argmax_kernel<kW_Q1_0, false>, gemv_tern_argmax_kernel<kW_Q1_0, true>)
+                  : g.type == kW_PQ2_0
+                      ? pick(gemv_tern_argmax_kernel<kW_PQ2_0, false>, gemv_tern_argmax_kernel<kW_PQ2_0, true>)
+                      : pick(gemv_tern_argmax_kernel<kW_PTQ1_0, false>, gemv_tern_argmax_kernel<kW_PTQ1_0, true>);
   const int res = resident_blocks(k, (uint32_t)gemv_tern_lds_bytes(g.K), 64 * nw);
   const int ntiles = (g.N + 15) / 16;
   return ntiles < res ? ntiles : res;
@@ -6879,9 +6884,9 @@ hipError_t launch_argmax_fused(const GemvArgs &g, const FuseArgs &f, hipStream_t
     return hipGetLastError();
   };
   switch (g.type) {
-    case kW_Q1_0: return go(gemv_tern_argmax_kernel<kW_Q1_0>, tm::waves<kW_Q1_0>());
-    case kW_PQ2_0: return go(gemv_tern_argmax_kernel<kW_PQ2_0>, tm::waves<kW_PQ2_0>());
-    case kW_PTQ1_0: return go(gemv_tern_argmax_kernel<kW_PTQ1_0>, tm::waves<kW_PTQ1_0>());
+    case kW_Q1_0: return go(g.rotate ? gemv_tern_argmax_kernel<kW_Q1_0, true> : gemv_tern_argmax_kernel<kW_Q1_0, false>, tm::waves<kW_Q1_0>());
+    case kW_PQ2_0: return go(g.rotate ? gemv_tern_argmax_kernel<kW_PQ2_0, true> : gemv_tern_argmax_kernel<kW_PQ2_0, false>, tm::waves<kW_PQ2_0>());
+    case kW_PTQ1_0: return go(g.rotate ? gemv_tern_argmax_kernel<kW_PTQ1_0, true> : gemv_tern_argmax_kernel<kW_PTQ1_0, false>, tm::waves<kW_PTQ1_0>());
     case kW_Q6_K: return launch_kq_argmax<kW_Q6_K>(g, f, stream, ev, done);
     case kW_Q4_K: return launch_kq_argmax<kW_Q4_K>(g, f, stream, ev, done);
     default: return blk_argmax(g, f, stream, ev, done, nullptr);
@@ -6905,9 +6910,9 @@ hipError_t launch_tern_sample(const GemvArgs &g, const FuseArgs &f, hipStream_t 
   const int blocks = tern_sample_grid(g);
   if (blocks != f.blocks) return hipErrorInvalidValue;   // the workspace was sized for another grid
   switch (g.type) {
-    case kW_Q1_0: return go(gemv_tern_sample_kernel<kW_Q1_0>, tm::waves<kW_Q1_0>(), blocks);
-    case kW_PQ2_0: return go(gemv_tern_sample_kernel<kW_PQ2_0>, tm::waves<kW_PQ2_0>(), blocks);
-    case kW_PTQ1_0: return go(gemv_tern_sample_kernel<kW_PTQ1_0>, tm::waves<kW_PTQ1_0>(), blocks);
+    case kW_Q1_0: return go(g.rotate ? gemv_tern_sample_kernel<kW_Q1_0, true> : gemv_tern_sample_kernel<kW_Q1_0, false>, tm::waves<kW_Q1_0>(), blocks);
+    case kW_PQ2_0: return go(g.rotate ? gemv_tern_sample_kernel<kW_PQ2_0, true> : gemv_tern_sample_kernel<kW_PQ2_0, false>, tm::waves<kW_PQ2_0>(), blocks);
+    case kW_PTQ1_0: return go(g.rotate ? gemv_tern_sample_kernel<kW_PTQ1_0, true> : gemv_tern_sample_kernel<kW_PTQ1_0, false>, tm::waves<kW_PTQ1_0>(), blocks);
     default: return hipErrorInvalidValue;
   }
 }
@@ -7039,9 +7044,12 @@ hipError_t prepare_kernels() {
                                hipFuncAttributeMaxDynamicSharedMemorySize, mid_smem)) != hipSuccess)
     return e;
   {
-    const void *tk[3] = {reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_Q1_0>),
-                         reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_PQ2_0>),
-                         reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_PTQ1_0>)};
+    const void *tk[6] = {reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_Q1_0, false>),
+                         reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_PQ2_0, false>),
+                         reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_PTQ1_0, false>),
+                         reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_Q1_0, true>),
+                         reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_PQ2_0, true>),
+                         reinterpret_cast<const void *>(&gemv_tern_sample_kernel<kW_PTQ1_0, true>)};
     for (const void *fk : tk)
       if ((e = hipFuncSetAttribute(fk, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)tern_sample_lds_bytes(kGemvMaxK, 16))) != hipSuccess)
@@ -7056,9 +7064,12 @@ hipError_t prepare_kernels() {
       if ((e = hipFuncSetAttribute(kk[i], hipFuncAttributeMaxDynamicSharedMemorySize, (int)kl[i])) !=
           hipSuccess)
         return e;
-    const void *ak[3] = {reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_Q1_0>),
-                         reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_PQ2_0>),
-                         reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_PTQ1_0>)};
+    const void *ak[6] = {reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_Q1_0, false>),
+                         reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_PQ2_0, false>),
+                         reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_PTQ1_0, false>),
+                         reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_Q1_0, true>),
+                         reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_PQ2_0, true>),
+                         reinterpret_cast<const void *>(&gemv_tern_argmax_kernel<kW_PTQ1_0, true>)};
     for (const void *fk : ak)
       if ((e = hipFuncSetAttribute(fk, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)gemv_tern_lds_bytes(kGemvMaxK))) != hipSuccess)

@@ -160,8 +160,10 @@ template <> struct TernSlot<kW_PTQ1_0> { static constexpr int kDepth = 2; uint32
 // (the sum over rounds, then over the four lane groups, in that fixed
 // order) go to epi.out(lane, row, value, valid) from every lane of one wave
 // at once (lanes 0..15 hold them; the point is wave-uniform).  The LDS from
-// `tlds` on holds gemv_tern_lds_bytes(K).
-template <int FMT, typename Epi>
+// `tlds` on holds gemv_tern_lds_bytes(K).  ROT: a Hadamard-folded weight, x
+// is rotated here first (kernels of their own: the switch at run time cost
+// the plain GEMVs 3 %).
+template <int FMT, bool ROT, typename Epi>
 __device__ __forceinline__ void tern_gemv_body(const GemvArgs &g, uint4 *tlds, Epi &epi) {
   using tm::v4i;
   constexpr int QB = tern_quant_bytes(FMT);
@@ -270,11 +272,25 @@ __device__ __forceinline__ void tern_gemv_body(const GemvArgs &g, uint4 *tlds, E
   constexpr int kPre = D < 2 ? D : 2;
   const float *xm = g.x + (int64_t)m * g.ldx;
   float xv[XB][2];
+  float rv[8];   // a Hadamard-folded weight: wave w's 512 inputs, 512 w + 64 i + lane
+  static_assert(NWV * 512 >= kGemvMaxK, "a wave for every 512 inputs");
+  const bool rot_wave = ROT && 512 * wave < K;
+  if constexpr (ROT) {
+    if (rot_wave) {
 #pragma unroll
-  for (int k = 0; k < XB; ++k) {
-    const int b = wave + k * NWV;
-    xv[k][0] = b < nb ? xm[128 * b + lane] : 0.f;
-    xv[k][1] = b < nb ? xm[128 * b + 64 + lane] : 0.f;
+      for (int i = 0; i < 8; ++i) {
+        const int p = 512 * wave + 64 * i + lane;
+        rv[i] = xm[p];
+        if (g.signs) rv[i] = rv[i] * g.signs[p];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < XB; ++k) {
+      const int b = wave + k * NWV;
+      xv[k][0] = b < nb ? xm[128 * b + lane] : 0.f;
+      xv[k][1] = b < nb ? xm[128 * b + 64 + lane] : 0.f;
+    }
   }
   TernSlot<FMT> slot[D];
   int c0 = 0, ct = 1, i0 = 0, n = 0;
@@ -286,6 +302,46 @@ __device__ __forceinline__ void tern_gemv_body(const GemvArgs &g, uint4 *tlds, E
   for (int u = 0; u < kPre; ++u) {
     load(c0, lt0, lr0, slot[u], u < n);
     if (++lt0 == ct) { lt0 = 0; ++lr0; }
+  }
+
+  // ---- the rotation of src/kernels.ts:177-227 (mode 0), a wave per 512: the
+  // butterfly stages over pairs (p, p + h), h = 1 .. 32 between lanes, 64 ..
+  // 256 in registers, each value the same binary32 sum or difference as
+  // hadamard_kernel's, then binary32(1 / sqrt(512)); the rotated x passes
+  // through the LDS of the partial results.  (Bound by its latency: as a
+  // launch of its own, Q1_0 151936 x 2048 took 20.8 us, now 18.3; PQ2_0 x 4096
+  // 40.6, now 38.5; unrotated 15.8 and 35.4.)
+  if constexpr (ROT) {
+    if (rot_wave) {
+#pragma unroll
+      for (int h = 1; h < 64; h <<= 1) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float o = __shfl_xor(rv[i], h);
+          rv[i] = lane & h ? o - rv[i] : rv[i] + o;
+        }
+      }
+#pragma unroll
+      for (int h = 1; h < 8; h <<= 1) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if (i & h) continue;
+          const float a = rv[i], b = rv[i + h];
+          rv[i] = a + b;
+          rv[i + h] = a - b;
+        }
+      }
+      const float norm = 0.04419417382415922f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) part[512 * wave + 64 * i + lane] = rv[i] * norm;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < XB; ++k) {
+      const int b = wave + k * NWV;
+      xv[k][0] = b < nb ? part[128 * b + lane] : 0.f;
+      xv[k][1] = b < nb ? part[128 * b + 64 + lane] : 0.f;
+    }
   }
 
   // ---- the tables of activation row m, once per workgroup: each block's
