@@ -1647,7 +1647,8 @@ __device__ __forceinline__ void finish_row(const LaunchArgs &a, const RowPlan &P
             ChaseSmem &cs = *reinterpret_cast<ChaseSmem *>(s.big + s.big_words);
             int lo = pick, hi = pick + 1;
             while (lo > 0 && pick - lo < kChaseMembers && s.skey[lo - 1] == kp) --lo;
-            while (hi < n && hi - pick < kChaseMembers && s.skey[hi] == kp) ++hi;
+            // (one past the limit, so that a group that goes on has g above it)
+            while (hi < n && hi - pick <= kChaseMembers && s.skey[hi] == kp) ++hi;
             const int g = hi - lo;
             if (tid < g && tid < kChaseMembers) cs.mem[tid] = s.sids[lo + tid];
             __syncthreads();   // (the arrays are the list's from here)
