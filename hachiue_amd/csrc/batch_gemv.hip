@@ -966,7 +966,8 @@ struct F32Batch {
       for (int r = 0; r < 4; ++r) {
         const float a = acc[t][h][r], x = (D[h][0][r] + D[h][1][r]) - low[t][h][r];
         const float n = a + x;
-        low[t][h][r] = (n - a) - x;
+        // (an infinite sum has lost nothing: Inf - Inf would make it NaN)
+        low[t][h][r] = fabsf(n) < __builtin_inff() ? (n - a) - x : 0.f;
         acc[t][h][r] = n;
       }
   }

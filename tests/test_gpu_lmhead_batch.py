@@ -1,7 +1,8 @@
 """GPU parity of the lm_head of several hidden states (batch_gemv.hip), where
 its slices and tiles end: M around 4, 8, 16, 32 and past the rows of one
-launch, N around a 16-row tile, the shortest and longest K.  The bound is the
-one of tests/test_gpu_lmhead.py, 2^-16 sum_k |x_k w_k| per logit."""
+launch, N around a 16-row tile, the shortest and longest K, within the bound
+of tests/test_gpu_lmhead.py, 2^-16 sum_k |x_k w_k| per logit.  Then rows that
+are not finite."""
 import numpy as np
 import pytest
 
@@ -52,18 +53,36 @@ def test_batched_rows_full_vocabulary(sampler, fmt):
 @pytest.mark.parametrize("fmt", list(ALL))
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
 def test_batched_row_with_non_finite_input(sampler, fmt, bad):
-    """The row of a non-finite element has no finite logit where its weight
-    is not 0, and is NaN everywhere on the integer formats; its neighbours are
-    untouched."""
+    """The row of a non-finite element is what it is in a call of its own, NaN
+    or an infinity in the same places (NaN everywhere on the integer formats);
+    its neighbours are untouched."""
     rng = np.random.default_rng(9)
     M, K, N = 11, 512, 300
     w = random_blocks(ALL[fmt], N, K, rng)
     x = rng.standard_normal((M, K)).astype(np.float32)
-    x[6, 300] = bad
+    x[6, 40] = bad                                  # (slabs follow it)
+    x[9, [3, 400]] = bad                            # both signs of it, by the weights
     y = run(sampler, fmt, x, w, N)
-    if fmt in ("f32", "q4_0", "q4_1"):
-        assert not np.isfinite(y[6]).any()
-    else:
-        assert np.isnan(y[6]).all()
-    keep = [r for r in range(M) if r != 6]
+    for r in (6, 9):
+        alone = run(sampler, fmt, x[[r]], w, N)[0]
+        assert not np.isfinite(alone).any()
+        if fmt != "q4_1":
+            assert np.array_equal(y[r], alone, equal_nan=True), (r, y[r, :8], alone[:8])
+        if fmt not in ("f32", "q4_1"):
+            assert np.isnan(y[r]).all()
+    keep = [r for r in range(M) if r not in (6, 9)]
     check(ALL[fmt], x[keep], w, N, y[keep])
+
+
+def test_batched_f32_sums_that_overflow(sampler):
+    """Finite inputs whose products or partial sums pass the largest binary32:
+    an infinity stays one through the slabs after it, as in a call of one row."""
+    rng = np.random.default_rng(10)
+    M, K, N = 5, 512, 200
+    w = rng.standard_normal((N, K)).astype(np.float32)
+    w[:, 5] = np.where(np.arange(N) % 2, 8.0, -8.0)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[2, 5] = 3e38
+    y = run(sampler, "f32", x, w.view(np.uint8), N)
+    assert np.array_equal(y[2], np.where(np.arange(N) % 2, np.inf, -np.inf).astype(np.float32))
+    assert np.isfinite(y[[0, 1, 3, 4]]).all()
