@@ -11,17 +11,27 @@
 // A weight of a super-block (256 positions) is d * w with w = sc * (q - 32)
 // (Q6_K, |w| <= 4096) or w = sc * q (Q4_K, at most 945, the minima apart): an
 // integer of 14 bits, held as two int8, w = 256 hi + lo.  x is held as four
-// int8 limbs per super-block, as in the one-row kernels (there per 16
-// positions): with 2^E above the block's largest |x|, a_t = rint(r_{t-1} *
-// 2^(6 + 7t - E)), r_t the exact remainder, |a_t| <= 64.  An A tile (16 x 64)
-// holds four limbs of four activation rows, A row 4 h + t limb t of row h; B
-// (64 x 16) one of the two bytes of 16 weight rows.  Eight MFMAs per
-// super-block and A tile (four steps of 64 positions, hi and lo) leave in
-// lane (j, h) of the result the four exact limb sums of (weight row j,
-// activation row h), in magnitude at most 2^26: one product per lane, so the
-// running binary32 sum of a tile takes one register per A tile.
+// int8 limbs per super-block: with 2^E above the block's largest |x|, x is
+// rounded to n 2^(E - 31) and the limbs are n's balanced base-256 digits a_t,
+// x = sum_t a_t 2^(E - 7 - 8t) to 2^(E - 32).  An A tile (16 x 64) holds four
+// limbs of four activation rows, A row 4 h + t limb t of row h; B (64 x 16)
+// one of the two bytes of 16 weight rows.  Eight MFMAs per super-block and A
+// tile (four steps of 64 positions, hi and lo) leave in lane (j, h) of the
+// result the four exact limb sums of (weight row j, activation row h), in
+// magnitude at most 2^27: one product per lane, so the running binary32 sum
+// of a tile takes one register per A tile.
 // (One row on the same instruction fills a quarter of an A tile with zeros
 // around its four limbs; four rows fill it.)
+//
+// The one-row kernels hold x to 2^(E_g - 28) with an exponent E_g for every
+// 16 positions (Q4_0 and Q4_1 hold it in binary32, and round at 2^-25 of a
+// block of 32).  Where a super-block's largest |x| is so far above a group's
+// that its limbs are coarser than that (E_g < E - 4; for Q4_0 and Q4_1 a
+// block's E_b < E - 7), the remainders of such groups become a second set of
+// four limbs with an exponent of its own, which a wave adds in a branch for
+// the super-blocks and A tiles that have one (outlier channels of 20 times
+// the rest and more).  The two sets are no coarser than one row's limbs
+// unless the small groups themselves lie more than 2^35 apart.
 //
 // The limbs are made by a kernel of their own (limbs_kernel) into the
 // context's workspace, laid out as the A operands are read; a workgroup
@@ -54,12 +64,13 @@ template <int FMT> struct Slab;
 template <> struct Slab<kW_Q6_K> {
   static constexpr int kBytes = 210;                     // of a row's super-block
   static constexpr int kChunks = q6m::kRowChunks;        // its 16-byte aligned cover
-  static constexpr int kRec = 16;                        // bytes of an activation row's record
+  // bytes of an activation row's record: 2^(E - 7), the second set's or 0
+  static constexpr int kRec = 16;
 };
 template <> struct Slab<kW_Q4_K> {
   static constexpr int kBytes = 144;
   static constexpr int kChunks = q4m::kRowChunks;
-  static constexpr int kRec = 48;                        // 2^(E - 6), then eight sums of x
+  static constexpr int kRec = 48;                        // and from byte 16 eight sums of x
 };
 template <> struct Slab<kW_Q4_0> {                        // eight blocks
   static constexpr int kBytes = 144;
@@ -208,13 +219,39 @@ __device__ __forceinline__ void decode(const uint8_t *rowb, uint32_t o, int G, B
 }
 }  // namespace bg
 
+namespace bg {
+// x to a multiple of 2^(E - 31), 2^E above the |x| of the wave's block: the
+// four balanced base-256 digits as bytes, most significant first from byte 3
+// down, and what is left of x (both exact)
+__device__ __forceinline__ uint32_t digits(float x, int E, float &rest) {
+  const float n = rintf(ldexpf(x, 31 - E));
+  rest = x - ldexpf(n, E - 31);
+  return ((uint32_t)(int)n + 0x80808080u) ^ 0x80808080u;
+}
+// E with |x| < 2^E for a largest |x| of mx, one more where the digits' largest
+// number, 0x7F7F7F7F, would be passed
+__device__ __forceinline__ int digits_exp(float mx) {
+  int E = 0;
+  (void)frexpf(mx, &E);
+  return E + (ldexpf(mx, 31 - E) >= 0x7F7F7F80p0f ? 1 : 0);
+}
+// limb t of four positions from their digits
+__device__ __forceinline__ uint32_t limb4(const uint32_t (&u)[4], int t) {
+  const uint32_t sel = (uint32_t)(3 - t) | (uint32_t)(7 - t) << 8;   // one byte of each of two
+  const uint32_t lo = __builtin_amdgcn_perm(u[1], u[0], sel), hi = __builtin_amdgcn_perm(u[3], u[2], sel);
+  return (lo & 0xFFFFu) | hi << 16;
+}
+}  // namespace bg
+
 // The A operands of activation rows 0..M-1: one wave per (super-block, row),
-// four positions a lane.  tab: [ceil(M / 4 ht)][K / 256][a_bytes(ht)].  A
-// block with a non-finite element gets a NaN scale, which makes every result
-// of its row NaN.
+// four positions a lane.  tab: [ceil(M / 4 ht)][K / 256][a_bytes(ht)], the
+// second sets' limbs in the same places from kBatchTabBytes on (written where
+// the record says that there is one).  A block with a non-finite element gets
+// a NaN scale, which makes every result of its row NaN.
 template <int FMT>
 __global__ __launch_bounds__(64) void limbs_kernel(const float *x, int64_t ldx, int NS, int ht,
                                                    uint8_t *tab) {
+  constexpr bool k32 = FMT == kW_Q4_0 || FMT == kW_Q4_1;
   const int s = (int)blockIdx.x, m = (int)blockIdx.y, lane = (int)threadIdx.x;
   const float *xp = x + (int64_t)m * ldx + 256 * s + 4 * lane;
   float v[4], mx = 0.f;
@@ -227,28 +264,33 @@ __global__ __launch_bounds__(64) void limbs_kernel(const float *x, int64_t ldx, 
   }
   double sum = ((double)v[0] + (double)v[1]) + ((double)v[2] + (double)v[3]);
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-#pragma unroll
   for (int o = 4; o > 0; o >>= 1) sum += __shfl_xor(sum, o);   // of the 32 positions of 8 lanes
   fin = __all(fin);
-  int E = 0;
-  (void)frexpf(fin ? mx : 1.f, &E);   // mx < 2^E
-  uint32_t limb[4] = {0u, 0u, 0u, 0u};
+  // the largest of the group that one row's limbs share an exponent in (16
+  // positions, 4 lanes; Q4_0 and Q4_1: of the block of 32), then of all
+  constexpr int GL = k32 ? 8 : 4;
+#pragma unroll
+  for (int o = 1; o < GL; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  int Eg = 0;
+  (void)frexpf(fin ? mx : 1.f, &Eg);
+#pragma unroll
+  for (int o = GL; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  const int E = bg::digits_exp(fin ? mx : 1.f);
+  const bool coarse = Eg < E - (k32 ? 7 : 4);
+  uint32_t u[4];
+  float rest[4], mr = 0.f;
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
-    float r = fin ? v[b] : 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float a = rintf(ldexpf(r, 6 + 7 * t - E));
-      r -= ldexpf(a, E - 6 - 7 * t);   // exact: a 2^(E-6-7t) is within half a step of r
-      limb[t] |= ((uint32_t)(int)a & 0xFFu) << (8 * b);
-    }
+    u[b] = bg::digits(fin ? v[b] : 0.f, E, rest[b]);
+    if (!coarse) rest[b] = 0.f;
+    mr = fmaxf(mr, fabsf(rest[b]));
   }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mr = fmaxf(mr, __shfl_xor(mr, o));
   // where the weights of position p sit in B: step and lane group (Q6_K:
   // p = 128 n + 32 step + 16 h + b in group 2 n + h, the quarters of a half
   // share their bytes; Q4_K: in order; Q4_0 and Q4_1, steps of 32: group G
   // has the low, then the high nibbles of bytes 4 G .. 4 G + 3)
-  constexpr bool k32 = FMT == kW_Q4_0 || FMT == kW_Q4_1;
   constexpr int W = k32 ? 8 : 16;   // bytes of a lane's A operand
   const int p = 4 * lane;
   const int step = k32 ? p >> 5 : FMT == kW_Q6_K ? (p >> 5) & 3 : p >> 6;
@@ -258,10 +300,25 @@ __global__ __launch_bounds__(64) void limbs_kernel(const float *x, int64_t ldx, 
   uint8_t *a = tab + ((int64_t)(m / (4 * ht)) * NS + s) * bg::a_bytes<FMT>(ht);
   uint8_t *d = a + (hid >> 2) * 4096 + step * 64 * W + (16 * G + 4 * (hid & 3)) * W + at;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) *reinterpret_cast<uint32_t *>(d + W * t) = limb[t];
+  for (int t = 0; t < 4; ++t) *reinterpret_cast<uint32_t *>(d + W * t) = bg::limb4(u, t);
+  float scale2 = 0.f;
+  if (mr > 0.f) {   // (uniform)
+    const int E2 = bg::digits_exp(mr);
+    scale2 = ldexpf(1.f, E2 - 7);
+    float lost;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) u[b] = bg::digits(rest[b], E2, lost);
+    d += kBatchTabBytes;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) *reinterpret_cast<uint32_t *>(d + W * t) = bg::limb4(u, t);
+  }
   float *rec = reinterpret_cast<float *>(a + ht * 4096 + hid * bg::Slab<FMT>::kRec);
-  if (lane == 0) rec[0] = fin ? ldexpf(1.f, E - 6) : __builtin_nanf("");
-  if (bg::Slab<FMT>::kRec > 16 && (lane & 7) == 0) rec[4 + (lane >> 3)] = (float)sum;
+  if (lane == 0) {
+    rec[0] = fin ? ldexpf(1.f, E - 7) : __builtin_nanf("");
+    rec[1] = scale2;
+  }
+  if (bg::Slab<FMT>::kRec > 16 && (lane & 7) == 0)   // (Q4_1: in units of the first limb's)
+    rec[4 + (lane >> 3)] = (float)(FMT == kW_Q4_1 ? ldexp(sum, 7 - E) : sum);
 }
 
 // Measured at 151936 x 2048, us a call, against one row at a time: Q1_0 4
@@ -394,6 +451,24 @@ __device__ __forceinline__ int batch_slice(int slices) { return ((int)blockIdx.x
 
 // ---- Q4_K and Q6_K
 
+namespace bg {
+// the four limb sums of a product, in units of the first limb's
+__device__ __forceinline__ float limb_sum(v4i d) {
+  float val = fmaf((float)d[3], 0x1p-8f, (float)d[2]);
+  val = fmaf(val, 0x1p-8f, (float)d[1]);
+  return fmaf(val, 0x1p-8f, (float)d[0]);
+}
+// bit r: row r of the slice (`rows` of them exist) has a second set of limbs
+// in the step whose records are at rec
+template <int FMT, int HT>
+__device__ __forceinline__ uint32_t second_rows(const uint8_t *rec, int lane, int rows) {
+  static_assert(4 * HT <= 32, "a bit a row");
+  float s = 0.f;
+  if (lane < 4 * HT && lane < rows) s = *reinterpret_cast<const float *>(rec + lane * Slab<FMT>::kRec + 4);
+  return (uint32_t)__builtin_amdgcn_ballot_w64(s > 0.f);
+}
+}  // namespace bg
+
 template <int FMT, int HT, int RT, bool HOLD>
 struct KqBatch {
   using S = bg::Slab<FMT>;
@@ -405,13 +480,15 @@ struct KqBatch {
   const v4i rw;
   uint32_t vo[kLoads];   // a lane's byte offset in a tile, per load
   const uint8_t *ab, *rec;
+  const uint8_t *second;   // the slice's second sets
+  uint32_t more;           // rows of the slice that have one in this step
   v4i A[HOLD ? HT : 1][4];
   float xs[HT];
   float acc[RT][HT];
 
-  __device__ __forceinline__ KqBatch(const GemvArgs &args, int sl)
+  __device__ __forceinline__ KqBatch(const GemvArgs &args, const uint8_t *tab, int sl)
       : g(args), slice(sl), lane(threadIdx.x & 63), j(lane & 15), G(lane >> 4),
-        rw(bg::rsrc(args.w, (args.w_bytes + 15u) & ~15u)) {}
+        rw(bg::rsrc(args.w, (args.w_bytes + 15u) & ~15u)), second(tab + kBatchTabBytes) {}
   // (rows at and past N lie past the resource, or wrap to its start: unused)
   __device__ __forceinline__ void at(int s) {
 #pragma unroll
@@ -437,6 +514,7 @@ struct KqBatch {
   __device__ __forceinline__ void step(const uint8_t *a) {
     ab = a;
     rec = a + HT * 4096;
+    more = bg::second_rows<FMT, HT>(rec, lane, g.M - slice * 4 * HT);
 #pragma unroll
     for (int h = 0; h < HT; ++h) {
       if constexpr (HOLD)
@@ -469,10 +547,7 @@ struct KqBatch {
         }
 #pragma unroll
       for (int h = 0; h < HP; ++h) {
-        const v4i dt = hi[h] * 256 + lw[h];
-        float val = fmaf((float)dt[3], 0x1p-7f, (float)dt[2]);
-        val = fmaf(val, 0x1p-7f, (float)dt[1]);
-        val = fmaf(val, 0x1p-7f, (float)dt[0]);
+        const float val = bg::limb_sum(hi[h] * 256 + lw[h]);
         const float ds = B.d * xs[h0 + h];   // d times a power of two
         if constexpr (FMT == kW_Q4_K) {   // the minima: - dmin sum_s m_s (sub-block s's sum of x)
           const float4 *xr = reinterpret_cast<const float4 *>(rec + (4 * (h0 + h) + G) * S::kRec + 16);
@@ -483,6 +558,22 @@ struct KqBatch {
         } else {
           acc[t][h0 + h] = fmaf(ds, val, acc[t][h0 + h]);
         }
+      }
+    }
+    if (__builtin_expect(more != 0u, 0)) {   // (wave-uniform; read from the table itself)
+      const uint8_t *a2 = second + (int64_t)s * kA + lane * 16;
+#pragma unroll
+      for (int h = 0; h < HT; ++h) {
+        if (!(more >> (4 * h) & 15u)) continue;
+        v4i hi = v4i{0, 0, 0, 0}, lw = hi;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const v4i a = *reinterpret_cast<const v4i *>(a2 + h * 4096 + k * 1024);
+          hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, B.hi[k], hi, 0, 0, 0);
+          lw = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, B.lo[k], lw, 0, 0, 0);
+        }
+        const float xs2 = *reinterpret_cast<const float *>(rec + (4 * h + G) * S::kRec + 4);
+        acc[t][h] = fmaf(B.d * xs2, bg::limb_sum(hi * 256 + lw), acc[t][h]);
       }
     }
   }
@@ -501,10 +592,10 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemv_batch_kq_kernel(GemvArgs
                                                                         int slices, int groups) {
   extern __shared__ uint4 blds[];
   const int slice = batch_slice(slices), NS = g.K / 256;
-  KqBatch<FMT, HT, RT, HOLD> body(g, slice);
-  batch_stream<KqBatch<FMT, HT, RT, HOLD>, RT, NW, NB>(
-      body, tab + (int64_t)slice * NS * bg::a_bytes<FMT>(HT), NS, g.N, slices, groups,
-      reinterpret_cast<uint8_t *>(blds));
+  tab += (int64_t)slice * NS * bg::a_bytes<FMT>(HT);
+  KqBatch<FMT, HT, RT, HOLD> body(g, tab, slice);
+  batch_stream<KqBatch<FMT, HT, RT, HOLD>, RT, NW, NB>(body, tab, NS, g.N, slices, groups,
+                                                       reinterpret_cast<uint8_t *>(blds));
 }
 
 // ---- Q1_0, PQ2_0, PTQ1_0: the codes are bytes as they are
@@ -778,7 +869,7 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemv_batch_tern_kernel(GemvAr
 // positions per block and A tile, B the block's q - 8 or q of 16 rows.  Lane
 // (j, G) takes the low, then the high nibbles of dword G of its row's block.
 // x as for the K-quants, limbs per 256 positions (eight blocks, one slab), so
-// 2^(E - 6) multiplies the slab's sum once.
+// 2^(E - 7) multiplies the slab's sum once.
 template <int FMT, int HT, int RT>
 struct Q4Batch {
   using S = bg::Slab<FMT>;
@@ -790,11 +881,13 @@ struct Q4Batch {
   const v4i rw;
   uint32_t vo[kLoads];
   const uint8_t *ab;
+  const uint8_t *second;   // as KqBatch's
+  uint32_t more;
   float acc[RT][HT];
 
-  __device__ __forceinline__ Q4Batch(const GemvArgs &args, int sl)
+  __device__ __forceinline__ Q4Batch(const GemvArgs &args, const uint8_t *tab, int sl)
       : g(args), slice(sl), lane(threadIdx.x & 63), j(lane & 15), G(lane >> 4),
-        rw(bg::rsrc(args.w, (args.w_bytes + 15u) & ~15u)) {}
+        rw(bg::rsrc(args.w, (args.w_bytes + 15u) & ~15u)), second(tab + kBatchTabBytes) {}
   __device__ __forceinline__ void at(int s) {
 #pragma unroll
     for (int c = 0; c < kLoads; ++c) {
@@ -813,12 +906,24 @@ struct Q4Batch {
 #pragma unroll
     for (int h = 0; h < HT; ++h) acc[t][h] = 0.f;
   }
-  __device__ __forceinline__ void step(const uint8_t *a) { ab = a; }
-  __device__ __forceinline__ void take(int t, int, int, const uint8_t *cur) {
+  __device__ __forceinline__ void step(const uint8_t *a) {
+    ab = a;
+    more = bg::second_rows<FMT, HT>(a + HT * 4096, lane, g.M - slice * 4 * HT);
+  }
+  // block b's q - 8 or q of this lane, low then high nibbles
+  static __device__ __forceinline__ int64_t quants(uint32_t q) {
+    uint32_t lo = q & 0x0F0F0F0Fu, hi = (q >> 4) & 0x0F0F0F0Fu;
+    if constexpr (FMT == kW_Q4_0) {   // q - 8 as a signed byte
+      lo = ((lo | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
+      hi = ((hi | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
+    }
+    return (int64_t)(((unsigned long long)hi << 32) | lo);
+  }
+  __device__ __forceinline__ void take(int t, int, int s, const uint8_t *cur) {
     const uint32_t *rowb = reinterpret_cast<const uint32_t *>(cur + j * 16 * S::kChunks);
     const uint8_t *rec = ab + HT * 4096;
-    float sum[HT], min[HT];   // the slab's, of d and (Q4_1) of m
-    uint32_t hd[8], q[8];     // d (and m); the lane group's dword
+    float sum[HT];          // the slab's
+    uint32_t hd[8], q[8];   // d (and m); the lane group's dword
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
       if constexpr (FMT == kW_Q4_0) {   // block b from byte 18 b: d, 16 bytes
@@ -833,33 +938,41 @@ struct Q4Batch {
     }
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      uint32_t lo = q[b] & 0x0F0F0F0Fu, hi = (q[b] >> 4) & 0x0F0F0F0Fu;
-      if constexpr (FMT == kW_Q4_0) {   // q - 8 as a signed byte
-        lo = ((lo | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-        hi = ((hi | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-      }
-      const int64_t B = (int64_t)(((unsigned long long)hi << 32) | lo);
+      const int64_t B = quants(q[b]);
       const float d = q6m::h2f(hd[b]);
 #pragma unroll
       for (int h = 0; h < HT; ++h) {
         const int64_t A = *reinterpret_cast<const int64_t *>(ab + h * 4096 + b * 512 + lane * 8);
         const v4i D = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B, v4i{0, 0, 0, 0}, 0, 0, 0);
-        float val = fmaf((float)D[3], 0x1p-7f, (float)D[2]);
-        val = fmaf(val, 0x1p-7f, (float)D[1]);
-        val = fmaf(val, 0x1p-7f, (float)D[0]);
-        sum[h] = b == 0 ? val * d : fmaf(val, d, sum[h]);
-        if constexpr (FMT == kW_Q4_1) {
+        const float val = bg::limb_sum(D);
+        if constexpr (FMT == kW_Q4_1) {   // (d q and m cancel within the block, as in a row alone)
           const float sx = *reinterpret_cast<const float *>(rec + (4 * h + G) * S::kRec + 16 + 4 * b);
-          const float m = q6m::h2f(hd[b] >> 16);
-          min[h] = b == 0 ? m * sx : fmaf(m, sx, min[h]);
+          const float w = fmaf(val, d, q6m::h2f(hd[b] >> 16) * sx);
+          sum[h] = b == 0 ? w : sum[h] + w;
+        } else {
+          sum[h] = b == 0 ? val * d : fmaf(val, d, sum[h]);
         }
       }
     }
 #pragma unroll
     for (int h = 0; h < HT; ++h) {
       const float xs = *reinterpret_cast<const float *>(rec + (4 * h + G) * S::kRec);
-      if constexpr (FMT == kW_Q4_1) acc[t][h] += min[h];
       acc[t][h] = fmaf(sum[h], xs, acc[t][h]);   // times a power of two
+    }
+    if (__builtin_expect(more != 0u, 0)) {
+      const uint8_t *a2 = second + (int64_t)s * kA + lane * 8;
+#pragma unroll
+      for (int h = 0; h < HT; ++h) {
+        if (!(more >> (4 * h) & 15u)) continue;
+        float sum2 = 0.f;
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+          const int64_t A = *reinterpret_cast<const int64_t *>(a2 + h * 4096 + b * 512);
+          const v4i D = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, quants(q[b]), v4i{0, 0, 0, 0}, 0, 0, 0);
+          sum2 = fmaf(bg::limb_sum(D), q6m::h2f(hd[b]), sum2);
+        }
+        acc[t][h] = fmaf(sum2, *reinterpret_cast<const float *>(rec + (4 * h + G) * S::kRec + 4), acc[t][h]);
+      }
     }
   }
   __device__ __forceinline__ void put(int t, int tile) {
@@ -878,9 +991,9 @@ __global__ __launch_bounds__(64 * NW, NW / 4) void gemv_batch_q4_kernel(GemvArgs
   extern __shared__ uint4 blds[];
   using Body = Q4Batch<FMT, HT, RT>;
   const int slice = batch_slice(slices), NS = g.K / 256;
-  Body body(g, slice);
-  batch_stream<Body, RT, NW, NB>(body, tab + (int64_t)slice * NS * Body::kA, NS, g.N, slices, groups,
-                                 reinterpret_cast<uint8_t *>(blds));
+  tab += (int64_t)slice * NS * Body::kA;
+  Body body(g, tab, slice);
+  batch_stream<Body, RT, NW, NB>(body, tab, NS, g.N, slices, groups, reinterpret_cast<uint8_t *>(blds));
 }
 
 // ---- F32: binary32 on v_mfma_f32_16x16x4_f32

@@ -792,7 +792,7 @@ int gemv_setup(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, const 
         (void)hipGetLastError();
         cs = hipStreamCaptureStatusActive;
       }
-      if (cs == hipStreamCaptureStatusNone) HS_HIP(ctx->gemv_tab.ensure(hs::kBatchTabBytes));
+      if (cs == hipStreamCaptureStatusNone) HS_HIP(ctx->gemv_tab.ensure(hs::kBatchWorkBytes));
     }
     g.tab = ctx->gemv_tab.p;
   }

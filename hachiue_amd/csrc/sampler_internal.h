@@ -280,10 +280,12 @@ constexpr int gemv_lds_bytes(int type) { return (kGemvThreads / 64) * gemv_batch
 hipError_t launch_gemv(const GemvArgs &g, hipStream_t stream, hipEvent_t *ev, hipEvent_t done);
 hipError_t prepare_gemv();      // per device, once (called by prepare_kernels)
 // Several activation rows in one pass over the weights (batch_gemv.hip), the
-// rows of one launch, and the bytes of their tables (16 slices of 16 rows,
-// K / 256 blocks of at most 17408 bytes each).
+// rows of one launch, the bytes of their tables (16 slices of 16 rows, K / 256
+// blocks of at most 17408 bytes each), and the workspace's: the tables, then
+// the second sets of limbs in the same places.
 constexpr int kBatchRows = 256;
 constexpr size_t kBatchTabBytes = (size_t)(kBatchRows / 16) * (kGemvMaxK / 256) * 17408;
+constexpr size_t kBatchWorkBytes = 2 * kBatchTabBytes;
 // From which M on: the K-quants, Q1_0 and PQ2_0 at once (2 rows 70 against 96
 // us, 22 against 29, 23 against 34); PTQ1_0 from 3 (2 rows take 42 us either
 // way, and greedy calls would lose their one launch); the others from 4 (one

@@ -1,11 +1,13 @@
 """GPU parity of the lm_head of several hidden states (batch_gemv.hip), where
 its slices and tiles end: M around 4, 8, 16, 32 and past the rows of one
 launch, N around a 16-row tile, the shortest and longest K, within the bound
-of tests/test_gpu_lmhead.py, 2^-16 sum_k |x_k w_k| per logit.  Then rows that
-are not finite."""
+of tests/test_gpu_lmhead.py, 2^-16 sum_k |x_k w_k| per logit.  Then what that
+bound does not see: the accuracy against a row at a time, and rows that are
+not finite."""
 import numpy as np
 import pytest
 
+from oracle import pyoracle as o
 from tests.test_gpu_lmhead import FORMATS, PLANAR, check, run_gemv, run_gemv_ex
 from tests.test_oracle_lmhead import random_blocks
 
@@ -86,3 +88,63 @@ def test_batched_f32_sums_that_overflow(sampler):
     y = run(sampler, "f32", x, w.view(np.uint8), N)
     assert np.array_equal(y[2], np.where(np.arange(N) % 2, np.inf, -np.inf).astype(np.float32))
     assert np.isfinite(y[[0, 1, 3, 4]]).all()
+
+
+# ---- accuracy: no coarser than a row at a time
+
+def without_channels(fmt, w, K, cols):
+    """The weights of the given channels set to 0 (of their sub-blocks too,
+    where a minimum is shared)."""
+    if fmt == "f32":
+        v = w.view(np.float32).reshape(-1, K).copy()
+        v[:, cols] = 0.0
+        return v.view(np.uint8)
+    B, BB = o.block_spec(ALL[fmt])
+    w = w.reshape(w.shape[0], K // B, BB).copy()
+    for c in cols:
+        blk, p = w[:, c // B], c % B          # (a view: written in place)
+        if fmt in ("q4_0", "q4_1"):           # q = 8; Q4_1's minimum is -8 d
+            i, hi = (2 if fmt == "q4_0" else 4) + p % 16, p >= 16
+            blk[:, i] = (blk[:, i] & 0x0F) | 0x80 if hi else (blk[:, i] & 0xF0) | 8
+            if fmt == "q4_1":
+                d = blk[:, 0:2].copy().view(np.float16)
+                blk[:, 2:4] = (d * np.float16(-8)).view(np.uint8)
+        elif fmt == "q4_k":                   # q = 0 and no minima in the super-block
+            i, hi = 16 + 32 * (p // 64) + p % 32, p % 64 >= 32
+            blk[:, i] &= 0x0F if hi else 0xF0
+            blk[:, 2:4] = 0
+        else:                                 # q6_k: q = 32
+            n, quarter, pos = p // 128, p % 128 // 32, p % 32
+            i, h = 64 * n + 32 * (quarter & 1) + pos, 128 + 32 * n + pos
+            blk[:, i] &= 0x0F if quarter >= 2 else 0xF0
+            blk[:, h] = (blk[:, h] & ~np.uint8(3 << 2 * quarter)) | np.uint8(2 << 2 * quarter)
+    return w.reshape(w.shape[0], -1)
+
+
+def error(fmt, x, w, N, y):
+    """Per row: rms error against binary64 over the logits' rms."""
+    exact, _ = o.gemv_exact(ALL[fmt], x, w, N)
+    e = y.astype(np.float64) - exact
+    return np.sqrt((e ** 2).mean(-1) / (exact ** 2).mean(-1))
+
+
+@pytest.mark.parametrize("fmt", ["f32", "q4_0", "q4_1", "q4_k", "q6_k"])
+@pytest.mark.parametrize("outlier", [1.0, 10.0, 1e3, 1e5, 1e8, 1e15])
+def test_batched_accuracy_with_outlier_channels(sampler, fmt, outlier):
+    """Hidden states with outlier channels whose weights are 0, so that all of
+    the signal lies in the small elements: the error against binary64 is not
+    above a row's own.  (Both are sums of binary32 values over 2048 products;
+    1.25 and 2^-24 allow for the order of their roundings.)"""
+    rng = np.random.default_rng(int(np.log10(outlier)) + 3)
+    M, K, N = 20, 2048, 1500
+    cols = [37, 700, 1301, 1999]
+    w = without_channels(fmt, random_blocks(ALL[fmt], N, K, rng), K, cols)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[:, cols] = (np.sign(x[:, cols]) * (0.5 + rng.random((M, len(cols)))) * outlier).astype(np.float32)
+    rows = np.array([0, 1, 2, 3, 6, 11, 19])
+    one = np.concatenate([error(fmt, x[[r]], w, N, run(sampler, fmt, x[[r]], w, N)) for r in rows])
+    for m in (M, 7, 4, 3, 2):
+        e = error(fmt, x[:m], w, N, run(sampler, fmt, x[:m], w, N))[rows[rows < m]]
+        ref = one[rows < m]
+        print(f"[accuracy] {fmt} outlier {outlier:g} M {m}: {e.mean():.2e}, one row {ref.mean():.2e}", flush=True)
+        assert (e <= 1.25 * ref + 2.0 ** -24).all(), (m, e, ref)
