@@ -975,13 +975,48 @@ struct Q4Batch {
       }
     }
   }
+  // A row's result in plain binary32, unit by unit as the one-row kernel
+  // forms them: what a row with a non-finite input is (the limbs, which
+  // cannot hold one, leave NaN; d q x + m x may be an infinity).
+  __device__ __forceinline__ float plain(int m, int row) const {
+    const float *x = g.x + (int64_t)m * g.ldx;
+    const uint32_t *w = static_cast<const uint32_t *>(g.w) + (int64_t)row * (g.row_bytes / 4u);
+    float r = 0.f;
+#pragma nounroll
+    for (int b = 0; b < g.K / 32 && r == r; ++b, x += 32, w += 5) {
+      float lo = 0.f, hi = 0.f, sum = 0.f;
+#pragma nounroll
+      for (int v = 0; v < 4; ++v) {
+        const uint32_t q4 = w[1 + v];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float xl = x[4 * v + i], xh = x[16 + 4 * v + i];
+          lo = fmaf(xl, (float)((q4 >> (8 * i)) & 15u), lo);
+          hi = fmaf(xh, (float)((q4 >> (8 * i + 4)) & 15u), hi);
+          sum += xl + xh;
+        }
+      }
+      r += fmaf(q6m::h2f(w[0]), lo + hi, q6m::h2f(w[0] >> 16) * sum);
+    }
+    return r;
+  }
   __device__ __forceinline__ void put(int t, int tile) {
-    const int row = tile * 16 + j;
+    const int row = tile * 16 + j, m0 = slice * 4 * HT + G;
+    uint32_t nan = 0;
 #pragma unroll
     for (int h = 0; h < HT; ++h) {
-      const int m = slice * 4 * HT + 4 * h + G;
-      if (row < g.N && m < g.M) g.y[(int64_t)m * g.ldy + row] = acc[t][h];
+      const int m = m0 + 4 * h;
+      if (row < g.N && m < g.M) {
+        g.y[(int64_t)m * g.ldy + row] = acc[t][h];
+        if (FMT == kW_Q4_1 && acc[t][h] != acc[t][h]) nan |= 1u << h;
+      }
     }
+    if constexpr (FMT == kW_Q4_1)
+      while (__builtin_expect(nan != 0u, 0)) {
+        const int m = m0 + 4 * (__ffs(nan) - 1);
+        g.y[(int64_t)m * g.ldy + row] = plain(m, row);
+        nan &= nan - 1u;
+      }
   }
 };
 

@@ -195,10 +195,11 @@ int hs_argmax(hs_context *ctx, const float *logits, int32_t rows,
  * 12 Q4_K, 14 Q6_K), N rows of K weights back to back, as the reference
  * uploads them (src/engine.ts:772-800).  K a multiple of the block size,
  * K <= 4096, W at most 4 GiB and 16-byte aligned.  Results differ from the
- * reference's binary32 sums by rounding only.  Q4_K and Q6_K (and Q4_0, Q4_1
- * from M = 4 on) run on the matrix cores with x held as integer limbs: a
- * non-finite element of an x row makes every result of that row NaN (the
- * reference's binary32 sums give NaN or +-Infinity there).  Several rows are
+ * reference's binary32 sums by rounding only.  Q4_K and Q6_K run on the
+ * matrix cores with x held as integer limbs: a non-finite element of an x row
+ * makes every result of that row NaN (the reference's binary32 sums give NaN
+ * or +-Infinity there; F32 and Q4_1 give what those sums give, Q4_0 NaN,
+ * since 8 times the block's sum of x is subtracted).  Several rows are
  * computed together where that reads the weights once; a row's results may
  * then differ by rounding from those of a call of its own.  Asynchronous on
  * `stream`. */

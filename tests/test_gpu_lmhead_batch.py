@@ -68,8 +68,7 @@ def test_batched_row_with_non_finite_input(sampler, fmt, bad):
     for r in (6, 9):
         alone = run(sampler, fmt, x[[r]], w, N)[0]
         assert not np.isfinite(alone).any()
-        if fmt != "q4_1":
-            assert np.array_equal(y[r], alone, equal_nan=True), (r, y[r, :8], alone[:8])
+        assert np.array_equal(y[r], alone, equal_nan=True), (r, y[r, :8], alone[:8])
         if fmt not in ("f32", "q4_1"):
             assert np.isnan(y[r]).all()
     keep = [r for r in range(M) if r not in (6, 9)]
