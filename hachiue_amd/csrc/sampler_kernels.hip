@@ -5787,9 +5787,10 @@ __global__ __launch_bounds__(kLT) void large_kernel(LaunchArgs a, Workspace ws) 
 //    parts stream it in rounds of kMpNV float4 per thread, two in flight.
 //  - Every wave keeps its own maximum m_w, raised before a round is summed
 //    (its sums are then scaled down), so no weight 2^((v - m_w) log2(e) / T)
-//    exceeds 1; they are added up in binary64.  The exponent is the binary32
-//    product with log2(e) / T as two binary32 parts, so that only roundings
-//    of its own, not one shared by the whole row, remain.
+//    exceeds 1; they are added up in binary64.  The weights are the general
+//    path's (exp_fast): the exponent in binary64, split into an integer and a
+//    rest for the hardware's exp2, so that none is off by more than that
+//    instruction's last place.
 //  - Logits at or above max so far + T ln(min_p) (a little less: kMpSlack)
 //    go to a list in LDS; the maximum is shared by the waves through LDS.
 //  - A part hands over its sums, its maximum and the listed logits that its
@@ -5863,13 +5864,13 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
   __syncthreads();
   const double it = 1.0 / P.temperature;
   const double cd = it * 1.4426950408889634074;   // log2(e) / T
-  const float ch = (float)cd, cl = (float)(cd - (double)ch);
   const float off = (float)((P.min_p < 1.0 ? log(P.min_p) * P.temperature : 0.0) - kMpSlack * P.temperature);
   // the list's bound for a maximum mx (the binary32 sum's rounding taken off)
   auto bound = [&](float mx) { return (mx + off) - 2.4e-7f * (fabsf(mx) + fabsf(off)); };
 
   float m_w = -INFINITY;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  double md = 0.0;   // m_w
+  double acc[2] = {0.0, 0.0};   // (four would be spilled)
   uint32_t nf = 0;
   auto append = [&](float v, int e, bool ok) {
     const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
@@ -5881,10 +5882,11 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
     if (ok && p < kMpCap) sm.list[p] = pack_cand(f2key(v), (uint32_t)e);
   };
   auto weigh = [&](float v, double &s) {
-    const float d = v - m_w;
-    // (NaN and -Infinity weigh 0: fmaxf gives the other operand for a NaN)
-    const float e = fmaxf(fmaf(d, ch, d * cl), -300.0f);
-    s += (double)__builtin_amdgcn_exp2f(e);
+    // (-Infinity and NaN weigh 2^-1000, nothing beside the maximum's 1: fmax
+    // gives the other operand for a NaN)
+    const double y = fmax(((double)v - md) * cd, -1000.0);
+    const double n = rint(y);
+    s += ldexp((double)__builtin_amdgcn_exp2f((float)(y - n)), (int)n);
     nf += v > -INFINITY ? 1u : 0u;
   };
   auto process = [&](f32x4 (&t)[kMpNV], int fb, float extra) {
@@ -5903,8 +5905,9 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
     if (wm > m_w) {
       const double f = m_w > -INFINITY ? exp(((double)m_w - (double)wm) * it) : 0.0;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[c] *= f;
+      for (int c = 0; c < 2; ++c) acc[c] *= f;
       m_w = wm;
+      md = (double)wm;
       if (lane == 0) atomicMax(&sm.mx, wk);
     }
     const float lo = bound(key2f(__builtin_amdgcn_readfirstlane(*(volatile uint32_t *)&sm.mx)));
@@ -5915,7 +5918,7 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
 #pragma unroll
     for (int u = 0; u < kMpNV; ++u) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) weigh(t[u][c], acc[c]);
+      for (int c = 0; c < 4; ++c) weigh(t[u][c], acc[c & 1]);
       const bool any = t[u][0] >= lo || t[u][1] >= lo || t[u][2] >= lo || t[u][3] >= lo;
       if (__builtin_expect(__any(any), 0)) {
         const int e = 4 * (f0 + fb + u * kRowThreads + tid);
@@ -5933,7 +5936,7 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
 
   // the part's sums: each wave's, scaled to the part's maximum
   {
-    double sw = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    double sw = acc[0] + acc[1];
     sw = wave_sum_f64(sw);
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) nf += __shfl_xor(nf, d);
@@ -6045,7 +6048,9 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
     }
     return true;
   }
-  if (bad || n < 1 || n > kSortCap || !(St > 0.0 && St < INFINITY) || !(mf < INFINITY)) return false;
+  // (the maximum weighs 1: a smaller sum lost it, to a reciprocal of T that is
+  // infinite)
+  if (bad || n < 1 || n > kSortCap || !(St >= 0.5 && St < INFINITY) || !(mf < INFINITY)) return false;
   sort_binned<kRowThreads>(sm.srt, n, f2key(bound(mf)), sm.mkey, sm.cnt, sm.tmp);
   __syncthreads();
   double *cum = reinterpret_cast<double *>(sm.list);

@@ -6,6 +6,7 @@ differ (tests/gpu_util.py)."""
 import numpy as np
 import pytest
 
+from tests.gpu_util import run_gpu, run_oracle
 from tests.test_gpu_large import _check
 
 pytestmark = pytest.mark.gpu
@@ -98,3 +99,54 @@ def test_mixed_batch(ctx):
     for _ in range(2):
         _check(ctx, x, vocab, hist.reshape(-1), np.arange(rows + 1, dtype=np.int64) * 30, cfgs,
                rng.random(rows), 64, "min-p mixed", want_cands=False)
+
+
+def test_normaliser_of_a_heavy_tail(ctx):
+    """Rows whose mass lies mostly in 600,000 equal logits far below the
+    candidates, so that a weight's error does not average out, at a value
+    where an exponent rounded to binary32 would be off by most of half a unit
+    (up to 6e-7 of the weight), with a top-p 3e-7 above or below a cumulative
+    probability: the cutoff and the token are the oracle's.  (Weights within
+    2^-23, the probabilities' own rounding 2^-24: below the 3e-7.)"""
+    rng = np.random.default_rng(17)
+    rows, vocab = 24, 600003
+    x = np.zeros((rows, vocab), np.float32)
+    cfgs, u, cuts = [], [], []
+    for r in range(rows):
+        t = float(rng.uniform(0.5, 1.3))
+        top = np.float32(rng.uniform(7.0, 9.0))
+        tail = np.float32(0)
+        while True:
+            tail = np.float32(top - t * rng.uniform(11.2, 12.0))
+            y = float(np.float32(tail - top)) / t / np.log(2.0)
+            off = (float(np.float32(y)) - y) * np.log(2.0)
+            if abs(off) > 5e-7:
+                break
+        x[r] = tail
+        near = rng.choice(vocab, 6, replace=False)
+        x[r, near] = top - (t * np.array([0.0, 4.0, 4.2, 4.4, 4.6, 4.8])).astype(np.float32)
+        e = np.exp((x[r].astype(np.float64) - float(top)) / t).astype(np.float32).astype(np.float64)
+        p = (e[near] / e.sum()).astype(np.float32).astype(np.float64)
+        j = int(rng.integers(0, 5))
+        up = int(off < 0)         # where the rounded exponent is too small, so is the sum
+        c = np.cumsum(p)[j] * (1 + (3e-7 if up else -3e-7))
+        cfgs.append(dict(temperature=t, topK=INF, topP=c, minP=0.006))
+        cuts.append(j + 1 + up)
+        u.append(rng.uniform(0.02, 0.6))
+    got = run_gpu(ctx, x, vocab, None, None, cfgs, np.array(u), 64, want_cands=False)
+    want, _ = run_oracle(x, vocab, None, None, cfgs, np.array(u), 64)
+    assert want.cutoff.tolist() == cuts
+    assert got.cutoff.tolist() == cuts
+    assert got.tokens.tolist() == want.token.tolist()
+
+
+def test_small_temperatures(ctx):
+    """Temperatures whose reciprocal overflows a binary32 or a binary64."""
+    rng = np.random.default_rng(23)
+    vocab = 9001
+    temps = [1e-6, 1e-20, 1e-37, 1e-39, 1e-300, 1e-310, 5e-324, 1e6, 1e38, 1e300]
+    x = (rng.standard_normal((len(temps), vocab)) * 3).astype(np.float32)
+    x[:, 77] = x[:, 4000] = 20.0
+    cfgs = [dict(temperature=t, topK=INF, topP=0.9, minP=0.1) for t in temps]
+    _check(ctx, x, vocab, None, None, cfgs, rng.random(len(temps)), 64, "min-p temperatures",
+           want_cands=False)

@@ -51,6 +51,13 @@ def _run(sampler, noalloc, logits, ids, off, u, configs):
 TIES = [dict(temperature=1.0, topK=20000, topP=0.95),
         dict(temperature=0.8, topK=5000, topP=0.9),
         dict(temperature=0.7, topK=40, topP=0.9, repetitionPenalty=1.1)]
+# min-p without top-k: the general large-k kernel here, the min-p kernel in
+# the allocating entry point; with and without a top-p stop, beside others
+MINP = [dict(temperature=1.0, topK=0, topP=1.0, minP=0.05, repetitionPenalty=1.1),
+        dict(temperature=0.8, topK=0, topP=0.9, minP=0.01),
+        dict(temperature=1.5, topK=0, topP=1.0, minP=0.002),
+        dict(temperature=1.0, topK=5000, topP=1.0, minP=0.1),
+        dict(temperature=0.7, topK=40, topP=0.9, repetitionPenalty=1.1)]
 
 
 def test_noalloc_matches_the_allocating_entry_point(sampler):
@@ -58,6 +65,8 @@ def test_noalloc_matches_the_allocating_entry_point(sampler):
              (3, 151936, 2, [MIX[0]] * 3, False),          # split rows: 9 parts each
              (3, 151936, 2, [MIX[0]] * 3, False),          # same configs: no upload
              (40, 50000, 3, [MIX[(r * 7) % len(MIX)] for r in range(40)], False),
+             (25, 151936, 6, [MINP[r % len(MINP)] for r in range(25)], False),
+             (5, 70001, 7, MINP, True),
              (6, 151936, 4, [TIES[r % len(TIES)] for r in range(6)], True),
              (3, 60000, 5, [TIES[r % len(TIES)] for r in range(3)], True)]
     for rows, vocab, seed, configs, coarse in calls:
