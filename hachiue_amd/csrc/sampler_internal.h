@@ -135,7 +135,7 @@ struct MinpMeta {
   uint32_t mkey;             // key of m, 0: no logit above -Infinity
   uint32_t nf;               // logits above -Infinity
   int32_t count;             // candidates handed over, -1: too many
-  uint32_t pad;
+  uint32_t kmin;             // a key that none of them is below
 };
 static_assert(sizeof(MinpMeta) == 24, "MinpMeta layout");
 

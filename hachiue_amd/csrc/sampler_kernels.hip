@@ -4168,8 +4168,15 @@ __device__ __forceinline__ LargeLoc large_locate(const LargeRow &L, int mode, do
 // kReplayCands candidate positions, large_replay_dev_kernel (slots in device
 // memory) up to k = kReplayDevMaxK and kReplayDevCands positions; beyond
 // those the row reports HS_ROW_UNSUPPORTED.
+// `known`: the row's extremes and its finite count where a kernel has them
+// already; otherwise the first pass finds them.
+struct LargeStart {
+  uint32_t kmax, kmin;   // the largest key, one that none is below (0: not known)
+  int nf;
+};
 __device__ __forceinline__ void large_row(const LaunchArgs &a, const RowPlan &P, int row,
-                                          LargeSmem &sm, ReplayReq *req) {
+                                          LargeSmem &sm, ReplayReq *req,
+                                          const LargeStart *known = nullptr) {
   const int tid = threadIdx.x;
   if (tid == 0) req->need = 0;
   LargeRow L;
@@ -4180,19 +4187,28 @@ __device__ __forceinline__ void large_row(const LaunchArgs &a, const RowPlan &P,
 
   // 1. extremes and n_F.  A thread meets its logits in index order, so its
   // first maximum is kept by the strict comparison.
-  uint32_t bkey = 0, bidx = 0, kmin = 0xFFFFFFFFu, nf = 0;
-  large_pass(L, [&](int e, float v) {
-    const uint32_t key = f2key(v);
-    const bool gt = key > bkey;
-    bkey = gt ? key : bkey;
-    bidx = gt ? (uint32_t)e : bidx;
-    const uint32_t km = key ? key : 0xFFFFFFFFu;
-    kmin = km < kmin ? km : kmin;
-    nf += key != 0u;
-  });
-  const unsigned long long best = block_max_u64(bkey ? pack_cand(bkey, bidx) : 0ull, sm);
-  const uint32_t kmin_all = ~(uint32_t)block_max_u64((unsigned long long)(~kmin), sm);
-  const int n_f = (int)block_sum_u64(nf, sm);
+  unsigned long long best;
+  uint32_t kmin_all;
+  int n_f;
+  if (known && known->kmin != 0u) {
+    best = pack_cand(known->kmax, 0u);   // (its id matters to a single candidate only)
+    kmin_all = known->kmin;
+    n_f = known->nf;
+  } else {
+    uint32_t bkey = 0, bidx = 0, kmin = 0xFFFFFFFFu, nf = 0;
+    large_pass(L, [&](int e, float v) {
+      const uint32_t key = f2key(v);
+      const bool gt = key > bkey;
+      bkey = gt ? key : bkey;
+      bidx = gt ? (uint32_t)e : bidx;
+      const uint32_t km = key ? key : 0xFFFFFFFFu;
+      kmin = km < kmin ? km : kmin;
+      nf += key != 0u;
+    });
+    best = block_max_u64(bkey ? pack_cand(bkey, bidx) : 0ull, sm);
+    kmin_all = ~(uint32_t)block_max_u64((unsigned long long)(~kmin), sm);
+    n_f = (int)block_sum_u64(nf, sm);
+  }
   const int k = P.k;
   const int n = k < n_f ? k : n_f;
   const int cs = a.cand_stride;
@@ -5790,7 +5806,8 @@ __global__ __launch_bounds__(kLT) void large_kernel(LaunchArgs a, Workspace ws) 
 //    exceeds 1; they are added up in binary64.  The weights are the general
 //    path's (exp_fast): the exponent in binary64, split into an integer and a
 //    rest for the hardware's exp2, so that none is off by more than that
-//    instruction's last place.
+//    instruction's last place.  (Exponents in binary32 were up to 7e-7 of a
+//    weight off; 256 rows took 43 us with them.)
 //  - Logits at or above max so far + T ln(min_p) (a little less: kMpSlack)
 //    go to a list in LDS; the maximum is shared by the waves through LDS.
 //  - A part hands over its sums, its maximum and the listed logits that its
@@ -5799,14 +5816,20 @@ __global__ __launch_bounds__(kLT) void large_kernel(LaunchArgs a, Workspace ws) 
 //    reference's probabilities f32(f32(exp((v - m) / T)) / S), the min-p and
 //    top-p stops and the draw from it (src/sampler.ts:83-117).
 // A row this does not suit (more than kMpCap logits listed by a part or
-// kSortCap kept, an infinite maximum, a normaliser that is not finite,
-// candidate outputs) is finished by large_row instead, by the
-// same workgroup.
-// Bound: one read of the row; the general path reads it four to six times
-// with one workgroup per row.  50 rows x 151936, min-p 0.05, repetition 1.1:
-// 174 us a call before (the general path 161 us of it), 30 us now (pen_kernel
-// 6, this kernel 25).
-constexpr int kMpNV = 8;          // float4 per thread and round
+// kSortCap kept, an infinite maximum, a normaliser that is not finite, a
+// maximum of 2^26 T and more, candidate outputs) is finished by large_row
+// instead, by the same workgroup, which takes the extremes and the count from
+// here in place of its own first pass; once a part's list is full it looks
+// for these alone.
+// Bound: one read of the row at small batches, from about 100 rows on the
+// weights' binary64 instructions (8 of 12 a logit); the general path reads a
+// row four to six times with one workgroup.  us a call at 151936 ids, general
+// path and now, min-p 0.05: 1 row 161, 20; 50 rows 167, 26; 256 rows 200, 49;
+// 1024 rows 737, 172.  Rows handed to large_row (flat logits, T 2, min-p
+// 0.02): 1 row 209, 197; 50 rows 242, 238; 256 rows 268, 262; 1024 rows 998,
+// 1010; the worst seen, rows of a few more candidates than are sorted, 221,
+// 230 at 256 rows.  So min_p alone decides the route (kMinpLeast).
+constexpr int kMpNV = 6;          // float4 per thread and round (8: spilled registers)
 constexpr int kMpCap = 4096;      // logits a part lists
 constexpr double kMpSlack = 1e-5; // of T, below the bound (probabilities round at 2^-24)
 
@@ -5816,9 +5839,10 @@ struct MinpSmem {
   unsigned long long tmp[kSortCap];
   uint32_t cnt[kBinSortBins + 32];
   double dred[kRowWaves];
-  uint32_t wkey[kRowWaves], wnf[kRowWaves];
+  uint32_t wkey[kRowWaves], wmin[kRowWaves], wnf[kRowWaves];
   double s;                          // the part's, then the row's normaliser
-  uint32_t mkey, nf;                 // its maximum (key), logits above -Infinity
+  uint32_t mkey, kmin, nf;           // its maximum (key), a key that none above -Infinity
+                                     //   is below, the number of those
   uint32_t mx;                       // largest key seen so far by any wave
   int32_t nlist, nsrt, last, bad, f1, f2, pick;
   int32_t pcnt[kSplitMax];           // the parts' list lengths
@@ -5862,16 +5886,26 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
     sm.f2 = sm.pick = 0x7FFFFFFF;
   }
   __syncthreads();
-  const double it = 1.0 / P.temperature;
-  const double cd = it * 1.4426950408889634074;   // log2(e) / T
-  const float off = (float)((P.min_p < 1.0 ? log(P.min_p) * P.temperature : 0.0) - kMpSlack * P.temperature);
+  // (wave-uniform: in scalar registers, as the round's logits take most of
+  // the others)
+  auto uniform = [](double x) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+  };
+  const double it = uniform(1.0 / P.temperature);
+  const double cd = uniform(it * 1.4426950408889634074);   // log2(e) / T
+  const float off = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(
+      (float)((P.min_p < 1.0 ? log(P.min_p) * P.temperature : 0.0) - kMpSlack * P.temperature))));
   // the list's bound for a maximum mx (the binary32 sum's rounding taken off)
   auto bound = [&](float mx) { return (mx + off) - 2.4e-7f * (fabsf(mx) + fabsf(off)); };
 
   float m_w = -INFINITY;
-  double md = 0.0;   // m_w
+  double mc = 0.0;   // - m_w log2(e) / T
   double acc[2] = {0.0, 0.0};   // (four would be spilled)
   uint32_t nf = 0;
+  float mn = has_tail ? vt : INFINITY;   // least logit
   auto append = [&](float v, int e, bool ok) {
     const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
     if (m == 0ull) return;
@@ -5882,18 +5916,30 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
     if (ok && p < kMpCap) sm.list[p] = pack_cand(f2key(v), (uint32_t)e);
   };
   auto weigh = [&](float v, double &s) {
-    // (-Infinity and NaN weigh 2^-1000, nothing beside the maximum's 1: fmax
-    // gives the other operand for a NaN)
-    const double y = fmax(((double)v - md) * cd, -1000.0);
-    const double n = rint(y);
-    s += ldexp((double)__builtin_amdgcn_exp2f((float)(y - n)), (int)n);
-    nf += v > -INFINITY ? 1u : 0u;
+    // (a weight below 2^-149 is nothing beside the maximum's 1; -Infinity and
+    // NaN weigh 0)
+    const double y = fma((double)v, cd, mc), n = rint(y);
+    const bool f = v > -INFINITY;
+    nf += f ? 1u : 0u;
+    s += (double)ldexpf(f ? __builtin_amdgcn_exp2f((float)(y - n)) : 0.f, (int)n);
+  };
+  // (as an atomic: a volatile read of LDS became a flat one, which waited for
+  // the next round's logits)
+  auto seen = [](const uint32_t *p) {
+    return __builtin_amdgcn_readfirstlane(
+        __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
   };
   auto process = [&](f32x4 (&t)[kMpNV], int fb, float extra) {
+    auto least = [&](const f32x4 &x) { mn = fminf(fminf(mn, fminf(x[0], x[1])), fminf(x[2], x[3])); };
     if (fb + kRound > n4) {   // the part's last round: reads past its end do not count
 #pragma unroll
-      for (int u = 0; u < kMpNV; ++u)
+      for (int u = 0; u < kMpNV; ++u) {
         if (fb + u * kRowThreads + tid >= n4) t[u] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+        else least(t[u]);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kMpNV; ++u) least(t[u]);
     }
     float lm = extra;
 #pragma unroll
@@ -5907,16 +5953,27 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
 #pragma unroll
       for (int c = 0; c < 2; ++c) acc[c] *= f;
       m_w = wm;
-      md = (double)wm;
+      mc = uniform(-(double)wm * cd);
       if (lane == 0) atomicMax(&sm.mx, wk);
     }
-    const float lo = bound(key2f(__builtin_amdgcn_readfirstlane(*(volatile uint32_t *)&sm.mx)));
+    // a list that is full: the row is large_row's, which needs the rest of
+    // the row for its extremes and count alone
+    if (__builtin_expect((int)seen(reinterpret_cast<const uint32_t *>(&sm.nlist)) > kMpCap, 0)) {
+      nf += extra > -INFINITY ? 1u : 0u;
+#pragma unroll
+      for (int u = 0; u < kMpNV; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) nf += t[u][c] > -INFINITY ? 1u : 0u;
+      return;
+    }
+    const float lo = bound(key2f(seen(&sm.mx)));
     if (__builtin_expect(__any(extra > -INFINITY), 0)) {
       weigh(extra, acc[0]);
       append(extra, et, extra >= lo);
     }
 #pragma unroll
     for (int u = 0; u < kMpNV; ++u) {
+      if (fb + u * kRowThreads >= n4) break;   // (uniform)
 #pragma unroll
       for (int c = 0; c < 4; ++c) weigh(t[u][c], acc[c & 1]);
       const bool any = t[u][0] >= lo || t[u][1] >= lo || t[u][2] >= lo || t[u][3] >= lo;
@@ -5945,11 +6002,14 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
       sm.wkey[wave] = f2key(m_w);
       sm.wnf[wave] = nf;
     }
+    // (-Infinity among the logits: the least that can be above it)
+    const uint32_t low = wave_max_u32(~f2key(fmaxf(mn, -FLT_MAX)));
+    if (lane == 0) sm.wmin[wave] = ~low;
   }
   __syncthreads();
   // (lanes 0 .. n - 1 of wave 0 hold partial sums s relative to key2f(k))
-  auto combine = [&](double s, uint32_t k, uint32_t c) {
-    const uint32_t mk = wave_max_u32(k);
+  auto combine = [&](double s, uint32_t k, uint32_t kmin, uint32_t c) {
+    const uint32_t mk = wave_max_u32(k), low = wave_max_u32(~kmin);
     double x = k ? s * exp(((double)key2f(k) - (double)key2f(mk)) * it) : 0.0;
     if (k == mk) x = s;   // (also where the difference is infinite minus itself)
     x = wave_sum_f64(k ? x : 0.0);
@@ -5958,12 +6018,15 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
     if (lane == 0) {
       sm.s = x;
       sm.mkey = mk;
+      sm.kmin = ~low;
       sm.nf = c;
     }
   };
-  if (wave == 0)
-    combine(lane < kRowWaves ? sm.dred[lane] : 0.0, lane < kRowWaves ? sm.wkey[lane] : 0u,
-            lane < kRowWaves ? sm.wnf[lane] : 0u);
+  if (wave == 0) {
+    const bool in = lane < kRowWaves;
+    combine(in ? sm.dred[lane] : 0.0, in ? sm.wkey[lane] : 0u, in ? sm.wmin[lane] : 0xFFFFFFFFu,
+            in ? sm.wnf[lane] : 0u);
+  }
   __syncthreads();
   const int nl = sm.nlist;
   bool bad = nl > kMpCap;
@@ -5992,6 +6055,7 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
       MinpMeta *m = ws.minp_meta + blockIdx.x;
       store_agent(&m->s, (unsigned long long)__double_as_longlong(sm.s));
       store_agent(&m->mkey, sm.mkey);
+      store_agent(&m->kmin, sm.kmin);
       store_agent(&m->nf, sm.nf);
       store_agent(&m->count, bad || sm.nsrt > kMinpHand ? -1 : sm.nsrt);
     }
@@ -6003,11 +6067,12 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
       const bool in = lane < S;
       const double s = in ? __longlong_as_double((long long)load_agent(&m0[lane].s)) : 0.0;
       const uint32_t k = in ? load_agent(&m0[lane].mkey) : 0u;
+      const uint32_t low = in ? load_agent(&m0[lane].kmin) : 0xFFFFFFFFu;
       const uint32_t c = in ? load_agent(&m0[lane].nf) : 0u;
       const int n = in ? load_agent(&m0[lane].count) : 0;
       if (in) sm.pcnt[lane] = n;
       const bool miss = __any(n < 0);
-      combine(s, k, c);
+      combine(s, k, low, c);
       if (lane == 0) {
         sm.bad = miss ? 1 : 0;
         sm.nsrt = 0;
@@ -6049,8 +6114,10 @@ __device__ __forceinline__ bool minp_row(const LaunchArgs &a, const Workspace &w
     return true;
   }
   // (the maximum weighs 1: a smaller sum lost it, to a reciprocal of T that is
-  // infinite)
-  if (bad || n < 1 || n > kSortCap || !(St >= 0.5 && St < INFINITY) || !(mf < INFINITY)) return false;
+  // infinite; and where m / T is large the exponents lose their last places)
+  if (bad || n < 1 || n > kSortCap || !(St >= 0.5 && St < INFINITY) || !(mf < INFINITY) ||
+      !(fabs((double)mf) * cd < 0x1p26))
+    return false;
   sort_binned<kRowThreads>(sm.srt, n, f2key(bound(mf)), sm.mkey, sm.cnt, sm.tmp);
   __syncthreads();
   double *cum = reinterpret_cast<double *>(sm.list);
@@ -6106,17 +6173,21 @@ __global__ __launch_bounds__(kRowThreads) void minp_kernel(LaunchArgs a, Workspa
   extern __shared__ unsigned long long ldyn[];
   __shared__ ReplayReq unused_req;   // k = vocab: never a replay
   const int slot = (int)blockIdx.x / a.minp_split, part = (int)blockIdx.x - slot * a.minp_split;
+  __shared__ LargeStart start;
+  if (threadIdx.x == 0) start.kmin = 0u;
   if (!a.want_cands) {   // (otherwise minp_split is 1)
     const int row = ws.minp_list[slot];
-    if (minp_row(a, ws, ws.plans[row], row, slot, part, *reinterpret_cast<MinpSmem *>(ldyn))) return;
-    __syncthreads();   // (uniform: the LDS is large_row's from here)
+    MinpSmem &sm = *reinterpret_cast<MinpSmem *>(ldyn);
+    if (minp_row(a, ws, ws.plans[row], row, slot, part, sm)) return;
+    if (threadIdx.x == 0 && sm.nf > 1u) start = LargeStart{sm.mkey, sm.kmin, (int)sm.nf};
   }
+  __syncthreads();   // (uniform: the LDS is large_row's from here)
   // (the plan is read again: kept from above it would cost registers, spilled)
   int again = slot;
   asm volatile("" : "+s"(again));
   const int row = ws.minp_list[again];
   const RowPlan P = ws.plans[row];
-  large_row(a, P, row, *reinterpret_cast<LargeSmem *>(ldyn), &unused_req);
+  large_row(a, P, row, *reinterpret_cast<LargeSmem *>(ldyn), &unused_req, &start);
 }
 
 // ---------------------------------------------------------------- GPU greedy route
