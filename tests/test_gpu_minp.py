@@ -140,6 +140,30 @@ def test_normaliser_of_a_heavy_tail(ctx):
     assert got.tokens.tolist() == want.token.tolist()
 
 
+def test_rows_handed_to_the_general_path(ctx):
+    """More candidates than the kernel sorts: the general path starts from the
+    extremes and the count found here, also where they come from a row whose
+    list was full early, with -Infinity and NaN among the logits, all above or
+    all below zero, and a maximum or minimum past the last whole float4."""
+    rng = np.random.default_rng(31)
+    rows, vocab = 10, 120003
+    x = (rng.standard_normal((rows, vocab)) * 0.7).astype(np.float32)
+    x[1, ::2] = -np.inf
+    x[2, ::3] = np.nan
+    x[3] += 15.0
+    x[4] -= 15.0
+    x[5, -1] = x[5].max() + 0.5
+    x[6, -1] = -40.0
+    x[7, 60000:] = -np.inf                              # whole parts without a logit
+    x[8] = np.round(x[8] * 4) / 4
+    x[9, 0], x[9, -1] = 3.4e38, -3.4e38
+    cfgs = [dict(temperature=1.0, topK=INF, topP=p, minP=m) for p, m in
+            [(1.0, 0.02), (0.9, 0.05), (1.0, 0.1), (0.8, 0.02), (1.0, 0.02), (1.0, 0.03), (0.5, 0.02),
+             (1.0, 0.02), (0.7, 0.02), (0.9, 0.05)]]
+    cfgs[9]["temperature"] = 1e38
+    _check(ctx, x, vocab, None, None, cfgs, rng.random(rows), 64, "min-p, handed over", want_cands=False)
+
+
 def test_small_temperatures(ctx):
     """Temperatures whose reciprocal overflows a binary32 or a binary64."""
     rng = np.random.default_rng(23)
