@@ -187,7 +187,9 @@ struct hs_context {
   DevBuf split_list, split_meta, split_cnt;   // split rows (split_cnt: zero between calls)
   DevBuf gemv_part, gemv_cnt;   // Q4_K/Q6_K GEMV tiles cut between waves (gemv_cnt: zero between calls)
   DevBuf gemv_rot;              // the Hadamard-rotated input of a folded weight (see gemv_setup)
-  DevBuf gemv_tab;              // limb tables of several activation rows (one size, for good)
+  DevBuf gemv_tab;              // limb tables of several activation rows (from creation on, in
+                                //   one size: a first call may be captured, and a captured
+                                //   graph's address stays good)
   DevBuf fuse_rows, fuse_pool, fuse_hist;   // lm_head GEMV that samples its rows: counters
                                 //   (zero between calls), the waves' two largest, the
                                 //   rows' key histograms (zero between calls)
@@ -782,20 +784,7 @@ int gemv_setup(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, const 
   const int64_t wpb = hs::kGemvThreads / 64;
   g.blocks = (int32_t)std::min<int64_t>((steps + wpb - 1) / wpb, 1 << 20);
   if (M > 65535) return fail(HS_ERR_UNSUPPORTED, "M %d above 65535", M);
-  if (hs::gemv_batched(w_type, M, K)) {
-    // several rows: their limb tables (one allocation of the largest size, so
-    // that a captured graph's address stays good).  A first call that is
-    // being captured cannot allocate and takes a row at a time.
-    if (!ctx->gemv_tab.p) {
-      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-      if (hipStreamIsCapturing(stream, &cs) != hipSuccess) {
-        (void)hipGetLastError();
-        cs = hipStreamCaptureStatusActive;
-      }
-      if (cs == hipStreamCaptureStatusNone) HS_HIP(ctx->gemv_tab.ensure(hs::kBatchWorkBytes));
-    }
-    g.tab = ctx->gemv_tab.p;
-  }
+  if (hs::gemv_batched(w_type, M, K)) g.tab = ctx->gemv_tab.p;   // several rows: their limb tables
   if (!g.tab && (w_type == hs::kW_Q6_K || w_type == hs::kW_Q4_K)) {   // the hand-over slots of tiles cut between waves
     int cus = 0;
     HS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
@@ -1171,6 +1160,7 @@ int hs_context_create(int device, hs_context **out) {
     ctx->na_last = new (std::nothrow) hs_sample_config[na::kMaxRows];
     if (!ctx->na_last) e = hipErrorOutOfMemory;
   }
+  if (e == hipSuccess) e = ctx->gemv_tab.ensure(hs::kBatchWorkBytes);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     hs_context_destroy(ctx);

@@ -4,9 +4,13 @@ launch, N around a 16-row tile, the shortest and longest K, within the bound
 of tests/test_gpu_lmhead.py, 2^-16 sum_k |x_k w_k| per logit.  Then what that
 bound does not see: the accuracy against a row at a time, and rows that are
 not finite."""
+import ctypes
+
 import numpy as np
 import pytest
 
+from hachiue_amd import Sampler, hip
+from hachiue_amd import sampler as hsamp
 from oracle import pyoracle as o
 from tests.test_gpu_lmhead import FORMATS, PLANAR, check, run_gemv, run_gemv_ex
 from tests.test_oracle_lmhead import random_blocks
@@ -147,3 +151,54 @@ def test_batched_accuracy_with_outlier_channels(sampler, fmt, outlier):
         ref = one[rows < m]
         print(f"[accuracy] {fmt} outlier {outlier:g} M {m}: {e.mean():.2e}, one row {ref.mean():.2e}", flush=True)
         assert (e <= 1.25 * ref + 2.0 ** -24).all(), (m, e, ref)
+
+
+# ---- graphs
+
+@pytest.mark.parametrize("fmt", ["q6_k", "pq2_0", "f32"])
+def test_first_call_captured(sampler, fmt):
+    """A context whose first batched call is being captured: the graph holds
+    the batched kernels, and each replay, with eager calls between, gives the
+    eager call's results bit for bit."""
+    R = hip.runtime()
+    vp = ctypes.c_void_p
+    R.hipStreamBeginCapture.argtypes = [vp, ctypes.c_int]
+    R.hipStreamEndCapture.argtypes = [vp, ctypes.POINTER(vp)]
+    R.hipGraphInstantiate.argtypes = [ctypes.POINTER(vp), vp, vp, vp, ctypes.c_size_t]
+    R.hipGraphLaunch.argtypes = [vp, vp]
+    R.hipGraphExecDestroy.argtypes = R.hipGraphDestroy.argtypes = [vp]
+    rng = np.random.default_rng(8)
+    M, K, N = 9, 1024, 5000
+    w = random_blocks(ALL[fmt], N, K, rng)
+    xs = [rng.standard_normal((M, K)).astype(np.float32) for _ in range(3)]
+    want = [run(sampler, fmt, x, w, N) for x in xs]
+    if fmt in PLANAR:
+        q, sc = hsamp.split_blocks(ALL[fmt], w)
+        d_w, d_s = hip.DeviceArray.from_numpy(q), hip.DeviceArray.from_numpy(sc)
+    else:
+        d_w, d_s = hip.DeviceArray.from_numpy(np.ascontiguousarray(w).reshape(-1)), None
+    wt = hsamp.weights(ALL[fmt], N, K, d_w.addr, d_s.addr if d_s else None, False, None)
+    d_x, d_y = hip.DeviceArray.from_numpy(xs[0]), hip.DeviceArray((M, N), np.float32)
+    d_y2 = hip.DeviceArray((M, N), np.float32)
+    st, graph, ex = hip.Stream(), vp(), vp()
+    print(f"[gpu] captured batched lm_head {fmt}", flush=True)
+    with Sampler(0) as ctx:
+        hip.check(R.hipStreamBeginCapture(st.handle, 0), "hipStreamBeginCapture")   # global mode
+        try:
+            ctx.gemv_device_ex(d_x.addr, M, K, wt, d_y.addr, N, stream=st)
+        finally:
+            hip.check(R.hipStreamEndCapture(st.handle, ctypes.byref(graph)), "hipStreamEndCapture")
+        hip.check(R.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, 0), "hipGraphInstantiate")
+        for x, y in zip(xs, want):
+            d_x.upload(x)
+            d_y.upload(np.zeros((M, N), np.float32))
+            hip.synchronize()
+            hip.check(R.hipGraphLaunch(ex, st.handle), "hipGraphLaunch")
+            st.synchronize()
+            assert np.array_equal(d_y.download().view(np.uint32), y.view(np.uint32))
+            ctx.gemv_device_ex(d_x.addr, M, K, wt, d_y2.addr, N, stream=st)
+            st.synchronize()
+            assert np.array_equal(d_y2.download().view(np.uint32), y.view(np.uint32))
+        R.hipGraphExecDestroy(ex)
+        R.hipGraphDestroy(graph)
+    st.destroy()
