@@ -104,6 +104,33 @@ def test_fused_full_vocabulary(sampler, fctx, unfused, fmt):
     assert np.array_equal(pen.view(np.uint32), pen2.view(np.uint32))
 
 
+@pytest.mark.parametrize("fmt", list(FUSED))
+def test_fused_each_row_alone(sampler, fctx, unfused, fmt):
+    """One row a call, which the one launch takes for every format and option
+    (several rows of most formats read the weights once and take two)."""
+    wtype, K, N = FUSED[fmt], 512, 70001
+    rng = np.random.default_rng(77 + wtype)
+    w = random_blocks(wtype, N, K, rng, scale=0.05)
+    fctx.set_timing(True)
+    try:
+        for r, cfg in enumerate(CFGS):
+            x = rng.standard_normal((1, K)).astype(np.float32)
+            hists = [rng.integers(0, N, 100)]
+            u = rng.random(1)
+            fctx.kernel_times()
+            tok, pen, ids, off = lm_head_sample(fctx, wtype, x, w, N, hists, [cfg], u)
+            t, calls = fctx.kernel_times()
+            assert calls == 1 and t["gemv_kernel"] > 0 and t["row_kernel"] == 0.0, (r, t)
+            raw, ref, res = expect(sampler, wtype, x, w, N, ids, off, [cfg], u)
+            assert np.array_equal(pen.view(np.uint32), ref.view(np.uint32))
+            assert tok[0] == res.token[0] or res.draw_margin[0] < 1e-6
+            tok2, pen2, _, _ = lm_head_sample(unfused, wtype, x, w, N, hists, [cfg], u)
+            assert tok.tolist() == tok2.tolist()
+            assert np.array_equal(pen.view(np.uint32), pen2.view(np.uint32))
+    finally:
+        fctx.set_timing(False)
+
+
 @pytest.mark.parametrize("fmt", ["q1_0", "q4_k", "q6_k"])
 @pytest.mark.parametrize("N", [1, 15, 17, 1000, 4099, 65537])
 def test_fused_small_and_ragged_vocabularies(sampler, fctx, N, fmt):
