@@ -40,12 +40,14 @@
 // tiles through a ring in LDS, as the one-row kernels do.
 //
 // What bounds it: up to 8 rows the weights' reads (151936 x 2048 Q6_K, 2
-// rows: 70 us a call, of which 3 us are limbs_kernel; one row at a time 96
-// us; 7 rows 75 and 284 us; Q4_K at K 4096, 7 rows 112 and 453 us), beyond
+// rows: 67 us a call, of which 3 us are limbs_kernel; one row at a time 94
+// us; 7 rows 69 and 276 us; Q4_K at K 4096, 7 rows 116 and 448 us), beyond
 // that the instructions of a tile: about 250 vector instructions to take it
 // apart, 13 per A tile to add its results up, 8 MFMAs per A tile (counters
 // at 64 rows: vector units busy 45 % of the cycles, matrix cores 31 %, hardly
-// overlapping).  16 rows 87 us (620 one at a time), 64 rows 199 us (2417).
+// overlapping).  16 rows 82 us (607 one at a time), 64 rows 219 us (2391).
+// With four outlier channels of 1000 times the rest, so that half the
+// super-blocks have a second set: 7 rows 76 us, 64 rows 276; Q4_K 7 rows 121.
 #include "sampler_internal.h"
 #include "kq_gemv.h"
 
@@ -322,10 +324,12 @@ __global__ __launch_bounds__(64) void limbs_kernel(const float *x, int64_t ldx, 
 }
 
 // Measured at 151936 x 2048, us a call, against one row at a time: Q1_0 4
-// rows 22 (55), 64 rows 109 (828); PQ2_0 4 rows 23 (63), 16 rows 40 (226);
-// PTQ1_0 4 rows 42 (80), 8 rows 46 (155); Q4_0 4 rows 50 (148), 64 rows 238
-// (2008); Q4_1 16 rows 80 (489); F32, K 1024, 4 rows 142 (432), 64 rows 205
-// (6877).  The errors against binary64 are no larger than one row's.
+// rows 20 (54), 64 rows 118 (828); PQ2_0 4 rows 23 (63), 16 rows 41 (226);
+// PTQ1_0 4 rows 40 (79), 8 rows 44 (155); Q4_0, K 1024, 4 rows 29 (86), 64
+// rows 125 (1220); Q4_1 4 rows 52 (137), 16 rows 81 (484); F32, K 1024, 4 rows
+// 149 (432), 64 rows 220 (6871).  Errors against binary64, K 2048, rms over
+// the logits' rms, and one row's: Q6_K 5.9e-8 (8.5e-8), Q4_K 6.9e-8 (9.0e-8),
+// Q4_0 8.2e-8 (2.3e-7), Q4_1 1.1e-7 (1.3e-7), F32 1.1e-7 (1.2e-7).
 
 // ---- the stream, shared by the formats
 //
@@ -1114,8 +1118,9 @@ struct F32Batch {
       for (int r = 0; r < 4; ++r) {
         const float a = acc[t][h][r], x = (D[h][0][r] + D[h][1][r]) - low[t][h][r];
         const float n = a + x;
-        // (an infinite sum has lost nothing: Inf - Inf would make it NaN)
-        low[t][h][r] = fabsf(n) < __builtin_inff() ? (n - a) - x : 0.f;
+        // (where the sum is infinite, Inf - Inf: any finite value does, and one
+        // that cannot overflow the next x)
+        low[t][h][r] = __builtin_amdgcn_fmed3f((n - a) - x, -0x1p100f, 0x1p100f);
         acc[t][h][r] = n;
       }
   }
