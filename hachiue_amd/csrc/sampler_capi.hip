@@ -196,7 +196,8 @@ struct hs_context {
   // HS_LMHEAD_FUSE at creation: 0 always two launches; 1 (default) one
   // launch for all-greedy calls on the planar, Q4_K and Q6_K weights; 2 also
   // for calls with k <= 64 sampling rows there and all-greedy calls on the
-  // vector-unit weights (F32, Q4_0, Q4_1)
+  // vector-unit weights (F32, Q4_0, Q4_1).  (Calls whose GEMV reads the
+  // weights once for several rows, gemv_batched: two launches always.)
   int fuse = 1;
   DevBuf minp_cand, minp_meta;  // split min-p rows' hand-over (counted in by split_cnt)
   DevBuf large_retry;           // two-pass large-k rows handed back
@@ -857,7 +858,8 @@ int gemv_device(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, const
 // their lengths in n[0..4], and in n[5] whether a row of the large list has
 // more slots than the LDS replay holds.  Routing as build_plans with every
 // row on the one-pass kernels (vocab <= kRowMaxVocab): rows with k <= 64
-// join the mid kernel's launch when it has rows.
+// join the mid kernel's launch when it has rows.  Min-p rows take the general
+// kernel here (the same answers, slower).
 void build_plans_fixed(const hs_sample_config *cfgs, int rows, int vocab, hs::RowPlan *plans,
                        int32_t *lists, int n[6]) {
   int n_pf = 0, n_row = 0, n_large = 0, n_mid = 0, n_small = 0, n_lfast = 0, big = 0;

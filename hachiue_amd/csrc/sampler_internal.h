@@ -286,11 +286,13 @@ hipError_t prepare_gemv();      // per device, once (called by prepare_kernels)
 constexpr int kBatchRows = 256;
 constexpr size_t kBatchTabBytes = (size_t)(kBatchRows / 16) * (kGemvMaxK / 256) * 17408;
 constexpr size_t kBatchWorkBytes = 2 * kBatchTabBytes;
-// From which M on: the K-quants, Q1_0 and PQ2_0 at once (2 rows 70 against 96
+// From which M on: the K-quants, Q1_0 and PQ2_0 at once (2 rows 67 against 94
 // us, 22 against 29, 23 against 34); PTQ1_0 from 3 (2 rows take 42 us either
 // way, and greedy calls would lose their one launch); the others from 4 (one
 // row at a time their greedy calls may run in one launch, whose sums are the
-// GEMV's bit for bit).
+// GEMV's bit for bit).  A call with several rows is then two launches under
+// every HS_LMHEAD_FUSE: the one launch has the one-row kernels' sums, and a
+// call's logits are those of the GEMV on the same rows, whatever the policy.
 constexpr bool gemv_batched(int type, int M, int K) {
   switch (type) {
     case kW_Q6_K: case kW_Q4_K: return M >= 2;

@@ -33,7 +33,8 @@
 //                    row's candidates, then the shared row completion.
 //   minp_kernel      rows with k = vocab and min-p: one pass, split like the
 //                    row kernel's rows.
-//   large_kernel     the other rows with k > 1024: one 1024-thread workgroup per row,
+//   large_kernel     the other rows with k > 1024 (and, for the entry point that
+//                    allocates nothing, the min-p rows): one 1024-thread workgroup per row,
 //                    several passes (radix select of the k-th value, softmax
 //                    normaliser, probability-mass histogram, positions located
 //                    by narrowing one bucket).
@@ -5778,7 +5779,8 @@ __device__ __forceinline__ bool large_fast(const LaunchArgs &a, const RowPlan &P
 }
 
 // Rows of lfast_list; a row it cannot finish is marked in large_retry for
-// large_kernel.  Calls that want candidate outputs are all handed back.  Four waves per SIMD: one workgroup per CU.
+// large_kernel.  Calls that want candidate outputs are all handed back.  Four
+// waves per SIMD: one workgroup per CU.
 __global__ __launch_bounds__(kFT, 4) void large_fast_kernel(LaunchArgs a, Workspace ws) {
   extern __shared__ unsigned long long ldyn[];
   const int row = ws.lfast_list[blockIdx.x];
