@@ -785,7 +785,7 @@ int gemv_setup(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, const 
   const int64_t wpb = hs::kGemvThreads / 64;
   g.blocks = (int32_t)std::min<int64_t>((steps + wpb - 1) / wpb, 1 << 20);
   if (M > 65535) return fail(HS_ERR_UNSUPPORTED, "M %d above 65535", M);
-  if (hs::gemv_batched(w_type, M, K)) g.tab = ctx->gemv_tab.p;   // several rows: their limb tables
+  if (hs::gemv_batched(w_type, M, N, K)) g.tab = ctx->gemv_tab.p;   // several rows: their limb tables
   if (!g.tab && (w_type == hs::kW_Q6_K || w_type == hs::kW_Q4_K)) {   // the hand-over slots of tiles cut between waves
     int cus = 0;
     HS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
@@ -1334,7 +1334,7 @@ int lm_head_sample(hs_context *ctx, const float *d_x, int32_t M, int64_t ldx, co
   const bool sample_ok = tern || w->type == hs::kW_Q6_K || w->type == hs::kW_Q4_K;
   // (several rows whose GEMV reads the weights once for all of them: two launches)
   bool fused = ctx->fuse && (sample_ok || ctx->fuse >= 2) && M > 0 && w->rows > 0 && configs &&
-               !hs::gemv_batched(w->type, M, w->cols) &&
+               !hs::gemv_batched(w->type, M, w->rows, w->cols) &&
                d_uniforms && d_tokens && (d_hist_ids == nullptr) == (d_hist_offsets == nullptr);
   std::vector<hs::RowPlan> plans;
   Routing rt;

@@ -286,20 +286,38 @@ hipError_t prepare_gemv();      // per device, once (called by prepare_kernels)
 constexpr int kBatchRows = 256;
 constexpr size_t kBatchTabBytes = (size_t)(kBatchRows / 16) * (kGemvMaxK / 256) * 17408;
 constexpr size_t kBatchWorkBytes = 2 * kBatchTabBytes;
-// From which M on: the K-quants, Q1_0 and PQ2_0 at once (2 rows 67 against 94
-// us, 22 against 29, 23 against 34); PTQ1_0 from 3 (2 rows take 42 us either
-// way, and greedy calls would lose their one launch); the others from 4 (one
-// row at a time their greedy calls may run in one launch, whose sums are the
-// GEMV's bit for bit).  A call with several rows is then two launches under
-// every HS_LMHEAD_FUSE: the one launch has the one-row kernels' sums, and a
-// call's logits are those of the GEMV on the same rows, whatever the policy.
-constexpr bool gemv_batched(int type, int M, int K) {
+// Whether M rows go together.  Their one pass takes two launches (about 12 us
+// at least) and whole tiles of 16 weight rows a wave, so it pays only where a
+// row at a time has enough to do, M N products of a row and some K.  us a
+// call, a row at a time and together, on both sides of each line:
+//   Q4_K    32000 x 2048, M 3 24, 27, M 4 31, 27; 64000 x 512, M 2 13, 15;
+//           8192 x 2048, M 16 28, 36 (more states a tile take longer)
+//   Q6_K    16000 x 4096, M 4 46, 51, M 6 67, 55; 32000 x 2048, M 3 31, 31, M 4
+//           41, 31; 4096 x 2048, M 32 38, 41
+//   Q1_0    M 2 96000 x 512 12.9, 13.4; 64000 x 4096 26, 20; M 16 500 x 512
+//   PQ2_0   10.4, 12.3, 4096 at every K less together
+//   PTQ1_0  M 2 equal at 151936 x 2048, and greedy calls would lose their one
+//           launch; M 3 16000 x 4096 31, 34; M 4 4096 x 2048 26, 22, x 4096 32, 34
+//   Q4_0    to M 3 greedy calls may run in one launch (with the one-row sums);
+//   Q4_1    M 4 500 x 2048 11, 17, 2000 x 2048 30, 22; M 16 500 x 512 10.6, 13.3
+//   F32     the same; M 4 4096 x 4096 89, 117; M 6 less together; M 16 500 x
+//           1024 20, 22, x 2048 38, 34 (and fewer than 256 weight rows, either
+//           format, M 256: 40 x 2048 47, 61)
+// A call with several rows together is two launches under every
+// HS_LMHEAD_FUSE: the one launch has the one-row kernels' sums, and a call's
+// logits are those of the GEMV on the same rows, whatever the policy.
+constexpr bool gemv_batched(int type, int M, int N, int K) {
+  const int64_t n = (int64_t)M * N;
   switch (type) {
-    case kW_Q6_K: case kW_Q4_K: return M >= 2;
-    case kW_Q1_0: case kW_PQ2_0: return M >= 2 && K % 512 == 0;
-    case kW_PTQ1_0: return M >= 3 && K % 512 == 0;
-    case kW_Q4_0: case kW_Q4_1: return M >= 4 && K % 256 == 0;
-    case kW_F32: return M >= 4 && K % 64 == 0;
+    case kW_Q4_K: return M >= 2 && n >= (M > 8 ? 240000 : K >= 1024 ? 120000 : 131072);
+    case kW_Q6_K: return M >= 2 && n >= (K > 2048 ? 96000 : M > 8 ? 160000 : 120000);
+    case kW_Q1_0: case kW_PQ2_0:
+      return K % 512 == 0 && (M == 2 ? (int64_t)N * K >= 90000000 : M > 2 && N >= 256 && n >= 10000);
+    case kW_PTQ1_0:
+      return K % 512 == 0 && (M == 3 ? N >= 32000 : M > 3 && n >= (M >= 16 || K <= 2048 ? 16000 : 20000));
+    case kW_Q4_0: case kW_Q4_1: return M >= 4 && K % 256 == 0 && n >= (K >= 2048 ? 8000 : 12288);
+    case kW_F32:
+      return M >= 4 && K % 64 == 0 && N >= 256 && n >= (M < 16 ? 24576 : K >= 2048 ? 8000 : 16000);
     default: return false;
   }
 }

@@ -43,6 +43,37 @@ def test_batched_rows(sampler, fmt, M, K, N):
     check(ALL[fmt], x, w, N, y)
 
 
+def batched_n(fmt, M, K):
+    """Weight rows from which on M rows go together (gemv_batched)."""
+    n = {"q4_k": (240000 if M > 8 else 131072) / M, "q6_k": (160000 if M > 8 else 120000) / M,
+         "q1_0": 90e6 / K if M == 2 else 10000 / M, "ptq1_0": 32000 if M == 3 else 20000 / M,
+         "q4_0": 12288 / M, "f32": (24576 if M < 16 else 16000) / M}
+    n["pq2_0"], n["q4_1"] = n["q1_0"], n["q4_0"]
+    return max(256, int(np.ceil(n[fmt])))
+
+
+@pytest.mark.parametrize("fmt", list(ALL))
+@pytest.mark.parametrize("M,K,extra", [(2, 1, 0), (3, 2, 1), (4, 0, 15), (5, 1, 16), (8, 4, 17), (9, 3, 5),
+                                       (16, 2, 33), (17, 1, 8), (32, 0, 3), (33, 2, 31), (64, 3, 7),
+                                       (259, 1, 2)])
+def test_rows_taken_together(sampler, fmt, M, K, extra):
+    """The batched kernels at the edges of their slices and of the rule that
+    takes them: from its least number of weight rows on, the last tile ragged
+    by `extra`.  Checked on the first, the last and some other weight rows."""
+    if M < {"ptq1_0": 3, "q4_0": 4, "q4_1": 4, "f32": 4}.get(fmt, 2):
+        pytest.skip("a row at a time")
+    K = K * STEP.get(fmt, 512) or 4096
+    N = batched_n(fmt, M, K) + extra
+    rng = np.random.default_rng(M * 1000 + K + extra)
+    w = random_blocks(ALL[fmt], N, K, rng)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[M // 2] *= np.exp2(rng.integers(-20, 20, K)).astype(np.float32)
+    x[-1, ::3] = 0.0
+    y = run(sampler, fmt, x, w, N, pad=3)
+    rows = np.unique(np.concatenate([np.arange(40), np.arange(N - 40, N), rng.integers(0, N, 200)]))
+    check(ALL[fmt], x, w[rows], len(rows), y[:, rows])
+
+
 @pytest.mark.parametrize("fmt", list(ALL))
 def test_batched_rows_full_vocabulary(sampler, fmt):
     rng = np.random.default_rng(5)
@@ -63,7 +94,7 @@ def test_batched_row_with_non_finite_input(sampler, fmt, bad):
     or an infinity in the same places (NaN everywhere on the integer formats);
     its neighbours are untouched."""
     rng = np.random.default_rng(9)
-    M, K, N = 11, 512, 300
+    M, K, N = 11, 512, 22003
     w = random_blocks(ALL[fmt], N, K, rng)
     x = rng.standard_normal((M, K)).astype(np.float32)
     x[6, 40] = bad                                  # (slabs follow it)
@@ -83,7 +114,7 @@ def test_batched_f32_sums_that_overflow(sampler):
     """Finite inputs whose products or partial sums pass the largest binary32:
     an infinity stays one through the slabs after it, as in a call of one row."""
     rng = np.random.default_rng(10)
-    M, K, N = 5, 512, 200
+    M, K, N = 5, 512, 5003
     w = rng.standard_normal((N, K)).astype(np.float32)
     w[:, 5] = np.where(np.arange(N) % 2, 8.0, -8.0)
     x = rng.standard_normal((M, K)).astype(np.float32)
@@ -141,7 +172,9 @@ def test_batched_accuracy_with_outlier_channels(sampler, fmt, outlier):
     would be an error of 2^-20 without outliers.)  The planar formats hold x as
     a row alone does."""
     rng = np.random.default_rng(int(np.log10(outlier)) + 3)
-    M, K, N = 20, 2048, 1500
+    M, K = 20, 2048
+    N = max(batched_n(fmt, m, K) for m in (20, 7, 4, 3, 2))
+    sub = rng.choice(N, 1500, replace=False)      # the weight rows looked at
     cols = [37, 700, 1301, 1999]
     w = random_blocks(ALL[fmt], N, K, rng)
     if fmt in FORMATS:
@@ -149,9 +182,14 @@ def test_batched_accuracy_with_outlier_channels(sampler, fmt, outlier):
     x = rng.standard_normal((M, K)).astype(np.float32)
     x[:, cols] = (np.sign(x[:, cols]) * (0.5 + rng.random((M, len(cols)))) * outlier).astype(np.float32)
     rows = np.array([0, 1, 2, 3, 6, 11, 19])
-    one = np.concatenate([error(fmt, x[[r]], w, N, run(sampler, fmt, x[[r]], w, N)) for r in rows])
+    alone = [run(sampler, fmt, x[[r]], w, N)[:, sub] for r in rows]
+    one = np.concatenate([error(fmt, x[[r]], w[sub], 1500, y) for r, y in zip(rows, alone)])
+    least = {"ptq1_0": 3, "q4_0": 4, "q4_1": 4, "f32": 4}.get(fmt, 2)
     for m in (M, 7, 4, 3, 2):
-        e = error(fmt, x[:m], w, N, run(sampler, fmt, x[:m], w, N))[rows[rows < m]]
+        y = run(sampler, fmt, x[:m], w, N)[:, sub]
+        # together or a row at a time, as the rule has it
+        assert np.array_equal(y[0], alone[0][0]) == (m < least), m
+        e = error(fmt, x[:m], w[sub], 1500, y)[rows[rows < m]]
         ref = one[rows < m]
         print(f"[accuracy] {fmt} outlier {outlier:g} M {m}: {e.mean():.2e}, one row {ref.mean():.2e}", flush=True)
         assert (e <= 1.25 * ref + 2.0 ** -24).all(), (m, e, ref)
@@ -172,7 +210,7 @@ def test_first_call_captured(sampler, fmt):
     R.hipGraphLaunch.argtypes = [vp, vp]
     R.hipGraphExecDestroy.argtypes = R.hipGraphDestroy.argtypes = [vp]
     rng = np.random.default_rng(8)
-    M, K, N = 9, 1024, 5000
+    M, K, N = 9, 1024, 17800
     w = random_blocks(ALL[fmt], N, K, rng)
     xs = [rng.standard_normal((M, K)).astype(np.float32) for _ in range(3)]
     want = [run(sampler, fmt, x, w, N) for x in xs]
