@@ -5845,8 +5845,9 @@ __global__ __launch_bounds__(kLT) void large_kernel(LaunchArgs a, Workspace ws) 
 // path and now, min-p 0.05: 1 row 161, 20; 50 rows 167, 26; 256 rows 200, 49;
 // 1024 rows 737, 172.  Rows handed to large_row (flat logits, T 2, min-p
 // 0.02): 1 row 209, 197; 50 rows 242, 238; 256 rows 268, 262; 1024 rows 998,
-// 1010; the worst seen, rows of a few more candidates than are sorted, 221,
-// 230 at 256 rows.  So min_p alone decides the route (kMinpLeast).
+// 1010; the worst seen over 1100 to 600000 ids and 1 to 1024 rows, 1024 such
+// rows of 32000 ids, 352, 377, and rows of a few more candidates than are
+// sorted, 221, 230 at 256 rows.  So min_p alone decides the route (kMinpLeast).
 constexpr int kMpNV = 6;          // float4 per thread and round (8: spilled registers)
 constexpr int kMpCap = 4096;      // logits a part lists
 constexpr double kMpSlack = 1e-5; // of T, below the bound (probabilities round at 2^-24)
