@@ -551,16 +551,17 @@ struct KqBatch {
         }
 #pragma unroll
       for (int h = 0; h < HP; ++h) {
-        const float val = bg::limb_sum(hi[h] * 256 + lw[h]);
-        const float ds = B.d * xs[h0 + h];   // d times a power of two
+        // times a power of two (d times that could pass the binary32 range
+        // where no product of x does)
+        const float val = bg::limb_sum(hi[h] * 256 + lw[h]) * xs[h0 + h];
         if constexpr (FMT == kW_Q4_K) {   // the minima: - dmin sum_s m_s (sub-block s's sum of x)
           const float4 *xr = reinterpret_cast<const float4 *>(rec + (4 * (h0 + h) + G) * S::kRec + 16);
           const float4 u = xr[0], v = xr[1];
           const float sa = fmaf(B.mf[1], u.y, B.mf[0] * u.x), sb = fmaf(B.mf[3], u.w, B.mf[2] * u.z);
           const float sc = fmaf(B.mf[5], v.y, B.mf[4] * v.x), sd = fmaf(B.mf[7], v.w, B.mf[6] * v.z);
-          acc[t][h0 + h] += fmaf(ds, val, -B.dmin * ((sa + sb) + (sc + sd)));
+          acc[t][h0 + h] += fmaf(B.d, val, -B.dmin * ((sa + sb) + (sc + sd)));
         } else {
-          acc[t][h0 + h] = fmaf(ds, val, acc[t][h0 + h]);
+          acc[t][h0 + h] = fmaf(B.d, val, acc[t][h0 + h]);
         }
       }
     }
@@ -577,7 +578,7 @@ struct KqBatch {
           lw = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, B.lo[k], lw, 0, 0, 0);
         }
         const float xs2 = *reinterpret_cast<const float *>(rec + (4 * h + G) * S::kRec + 4);
-        acc[t][h] = fmaf(B.d * xs2, bg::limb_sum(hi * 256 + lw), acc[t][h]);
+        acc[t][h] = fmaf(B.d, bg::limb_sum(hi * 256 + lw) * xs2, acc[t][h]);
       }
     }
   }

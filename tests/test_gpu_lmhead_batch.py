@@ -195,6 +195,28 @@ def test_batched_accuracy_with_outlier_channels(sampler, fmt, outlier):
         assert (e <= 1.25 * ref + 2.0 ** -24).all(), (m, e, ref)
 
 
+@pytest.mark.parametrize("fmt", ["q4_k", "q6_k"])
+def test_batched_outliers_near_the_binary32_range(sampler, fmt):
+    """Channels near the largest binary32 with weights of 0, block scales near
+    the largest binary16: the scale times the limbs' unit passes the range, no logit does,
+    here as in a row alone."""
+    rng = np.random.default_rng(21)
+    M, K = 6, 1024
+    N = batched_n(fmt, M, K)
+    cols = [9, 300, 1000]
+    w = without_channels(fmt, random_blocks(ALL[fmt], N, K, rng, scale=2e4), K, cols)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[1::2, cols] = 5e36
+    y = run(sampler, fmt, x, w, N)
+    sub = rng.choice(N, 300, replace=False)
+    for r in range(M):
+        alone = run(sampler, fmt, x[[r]], w, N)[0]
+        assert np.isfinite(alone).all() and np.isfinite(y[r]).all(), r
+        # (the groups of the huge channels lose their other elements, alone too)
+        if r % 2 == 0:
+            check(ALL[fmt], x[[r]], w[sub], 300, y[[r]][:, sub])
+
+
 # ---- graphs
 
 @pytest.mark.parametrize("fmt", ["q6_k", "pq2_0", "f32"])
